@@ -7,7 +7,7 @@
 // src/core/stream_gemm.cu:705-738), with one FP32 scale per 128x128 block, ws [N/128][K/128].
 //
 // Design:
-//  * One v_mfma_scale_f32_16x16x128_f8f6f4 per 16x16 output tile per 128-value K block: an MFMA covers exactly one
+//  * One v_mfma_f32_16x16x128_f8f6f4 per 16x16 output tile per 128-value K block: an MFMA covers exactly one
 //    scale block, so its FP32 result is scaled once and added to the accumulator (one FMA per output per
 //    block). Any permutation of K inside the block is harmless, since A and B use the same one.
 //  * Weights are the A operand (rows n) and activations the B operand (columns m). A workgroup (8 waves, 2 per
@@ -28,6 +28,7 @@
 
 #include <algorithm>
 #include <string>
+#include <type_traits>
 
 namespace lq {
 namespace {
@@ -49,6 +50,13 @@ constexpr int kStage = 2 * kOpBytes + kBM * 4;   // weights, activations, activa
 // conflicts; the former swizzle by row / 2 had them on half of all LDS cycles).
 __device__ __forceinline__ int swz(int row) { return (row & 7) ^ ((row >> 3) & 1); }
 __device__ __forceinline__ int lds_off(int row, int u) { return row * kRowBytes + ((u ^ swz(row)) << 4); }
+
+// The fragment of row `row` for lanes with K 32 t .. + 32 of a block.
+__device__ __forceinline__ i32x8 fragment(const uint8_t* op, int row, int t) {
+  const u32x4 lo = *reinterpret_cast<const u32x4*>(op + lds_off(row, 2 * t));
+  const u32x4 hi = *reinterpret_cast<const u32x4*>(op + lds_off(row, 2 * t + 1));
+  return i32x8{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
+}
 
 struct PrefillArgs {
   const uint8_t* xq;
@@ -83,6 +91,31 @@ __device__ __forceinline__ void dma4(__amdgpu_buffer_rsrc_t rs, uint8_t* lds, in
 // s_waitcnt with only vmcnt / lgkmcnt constrained (gfx9 encoding: vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8])
 #define LQ_WAIT_VM0() __builtin_amdgcn_s_waitcnt(0x0f70)
 #define LQ_WAIT_LGKM0() __builtin_amdgcn_s_waitcnt(0xc07f)
+
+// Four outputs of one token, columns n .. n + 3.
+template <bool BLOCK, int OUT>
+__device__ __forceinline__ void put_out(const PrefillArgs& a, int m, int n, f32x4 v) {
+  if constexpr (!BLOCK) v = f32x4{v[0] * a.alpha, v[1] * a.alpha, v[2] * a.alpha, v[3] * a.alpha};
+  const size_t o = static_cast<size_t>(m) * a.ldy + n;
+  if constexpr (OUT == kOutBf16) {
+    *reinterpret_cast<u32x2*>(static_cast<uint16_t*>(a.y) + o) =
+        u32x2{f32_to_bf16(v[0]) | (uint32_t(f32_to_bf16(v[1])) << 16),
+              f32_to_bf16(v[2]) | (uint32_t(f32_to_bf16(v[3])) << 16)};
+  } else {
+    f32x4* dst = reinterpret_cast<f32x4*>(static_cast<float*>(a.y) + o);
+    if constexpr (OUT == kOutF32Acc) {
+      const f32x4 old = *dst;
+      v = f32x4{old[0] + v[0], old[1] + v[1], old[2] + v[2], old[3] + v[3]};
+    }
+    *dst = v;
+  }
+}
+
+// A weight block's scale as a scalar load: `p` is uniform over the wave and constant during the launch. (As a vector
+// load it is counted with the loads to LDS, in order: its use waits for every operand load issued before it.)
+__device__ __forceinline__ float scalar_load(const float* p) {
+  return *reinterpret_cast<const __attribute__((address_space(4))) float*>(reinterpret_cast<uintptr_t>(p));
+}
 
 // BLOCK: the block-scaled form (each 128-value block's product scaled by its activation and weight scales and
 // folded into the accumulators); else one scale for the whole product, applied at the end, and the MFMAs
@@ -164,30 +197,25 @@ __global__ void __launch_bounds__(kThreads) prefill_fp8_kernel(const PrefillArgs
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  const float* wsrow = BLOCK ? a.ws + static_cast<size_t>((n0 >> 7) + wn) * a.KB : nullptr;
-  const bool wrows = n0 + wn * 128 < a.N;  // this wave's weight half exists
+  // (a weight half past the end takes the last one's scales: its outputs are never stored)
+  const float* wsrow = BLOCK ? a.ws + static_cast<size_t>(min((n0 >> 7) + wn, (a.N >> 7) - 1)) * a.KB : nullptr;
 
   // Fragment reads from an LDS stage: weight tile i (rows wn*128 + 16i + r) and token tile j (rows wm*64 + 16j
   // + r), 32 bytes at K 32t each.
-  auto frag = [&](const uint8_t* op, int row) {
-    const u32x4 lo = *reinterpret_cast<const u32x4*>(op + lds_off(row, 2 * t));
-    const u32x4 hi = *reinterpret_cast<const u32x4*>(op + lds_off(row, 2 * t + 1));
-    return i32x8{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
-  };
   i32x8 bf[4], af;
   float sc[4];
   f32x4 pr[4];
   // B fragments, the lane's four block scales and the first A fragment of K block kb (stage st)
-  auto block_start = [&](int st, int kb) {
+  float wnext = 0.f;  // the next block's weight scale, loaded a block ahead
+  auto block_start = [&](int st) {
     const uint8_t* sa = smem + st * kStage;
     const float* sxs = reinterpret_cast<const float*>(sa + 2 * kOpBytes);
-    const float wsc = (BLOCK && wrows) ? wsrow[kb] : 0.f;
-    af = frag(sa, wn * 128 + r);
+    af = fragment(sa, wn * 128 + r, t);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) bf[j] = frag(sa + kOpBytes, wm * 64 + 16 * j + r);
+    for (int j = 0; j < 4; ++j) bf[j] = fragment(sa + kOpBytes, wm * 64 + 16 * j + r, t);
     if constexpr (BLOCK) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) sc[j] = sxs[wm * 64 + 16 * j + r] * wsc;
+      for (int j = 0; j < 4; ++j) sc[j] = sxs[wm * 64 + 16 * j + r] * wnext;
     }
   };
   auto fold = [&](f32x4 (&dst)[4], const f32x4 (&p)[4], const float (&s)[4]) {
@@ -200,7 +228,8 @@ __global__ void __launch_bounds__(kThreads) prefill_fp8_kernel(const PrefillArgs
   issue(0, kb0);
   LQ_WAIT_VM0();
   __builtin_amdgcn_s_barrier();
-  block_start(0, kb0);
+  if (BLOCK) wnext = scalar_load(wsrow + kb0);
+  block_start(0);
   // Per K block and weight tile: the tile's four MFMAs, then the next tile's fragment read, then the fold of
   // the four results into the accumulators (the other wave on the SIMD issues its MFMAs meanwhile). The one
   // barrier per block sits after tile 7's MFMAs are issued: it publishes the next block's loads and frees this
@@ -212,17 +241,18 @@ __global__ void __launch_bounds__(kThreads) prefill_fp8_kernel(const PrefillArgs
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       if (i < 5 && kb + 1 < kb1) issue_part(st ^ 1, kb + 1, i);
+      if (BLOCK && i == 0) wnext = scalar_load(wsrow + min(kb + 1, a.KB - 1));
       // the tile's MFMAs at raised issue priority: the SIMD's other wave gets the slots between them for its
       // folds and fragment reads (measured 1-2 % faster than equal priority)
       __builtin_amdgcn_s_setprio(1);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        // E8M0 scale 127 = 1.0 on both operands: the plain FP8 x FP8 product of one 128-value block
+        // (scales 0: the compiler takes the unscaled instruction, which needs no scale load before it, 2 % faster)
         if constexpr (BLOCK)
-          pr[j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(af, bf[j], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 127,
-                                                                  0, 127);
+          pr[j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(af, bf[j], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 0,
+                                                                  0, 0);
         else
-          acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(af, bf[j], acc[i][j], 0, 0, 0, 127, 0, 127);
+          acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(af, bf[j], acc[i][j], 0, 0, 0, 0, 0, 0);
       }
       if constexpr (BLOCK)
         asm volatile("" ::"v"(pr[0]), "v"(pr[1]), "v"(pr[2]), "v"(pr[3]) : "memory");
@@ -230,7 +260,7 @@ __global__ void __launch_bounds__(kThreads) prefill_fp8_kernel(const PrefillArgs
         asm volatile("" ::"v"(acc[i][0]), "v"(acc[i][1]), "v"(acc[i][2]), "v"(acc[i][3]) : "memory");
       __builtin_amdgcn_s_setprio(0);
       if (i < 7) {
-        af = frag(sa, wn * 128 + 16 * (i + 1) + r);
+        af = fragment(sa, wn * 128 + 16 * (i + 1) + r, t);
       } else {
         // every wave's reads of this stage have returned and its loads of the next block have landed
         LQ_WAIT_LGKM0();
@@ -243,7 +273,7 @@ __global__ void __launch_bounds__(kThreads) prefill_fp8_kernel(const PrefillArgs
         asm volatile("" ::"v"(acc[i][0]), "v"(acc[i][1]), "v"(acc[i][2]), "v"(acc[i][3]));
       }
     }
-    if (kb + 1 < kb1) block_start(st ^ 1, kb + 1);
+    if (kb + 1 < kb1) block_start(st ^ 1);
   }
 
   if (part >= 0) {
@@ -303,21 +333,200 @@ __global__ void __launch_bounds__(kThreads) prefill_fp8_kernel(const PrefillArgs
     for (int i = 0; i < 8; ++i) {
       const int n = n0 + wn * 128 + 16 * i + 4 * t;
       if (n >= a.N) continue;
-      f32x4 v = acc[i][j];
-      if constexpr (!BLOCK) v = f32x4{v[0] * a.alpha, v[1] * a.alpha, v[2] * a.alpha, v[3] * a.alpha};
-      const size_t o = static_cast<size_t>(m) * a.ldy + n;
-      if constexpr (OUT == kOutBf16) {
-        *reinterpret_cast<u32x2*>(static_cast<uint16_t*>(a.y) + o) =
-            u32x2{f32_to_bf16(v[0]) | (uint32_t(f32_to_bf16(v[1])) << 16),
-                  f32_to_bf16(v[2]) | (uint32_t(f32_to_bf16(v[3])) << 16)};
-      } else {
-        f32x4* dst = reinterpret_cast<f32x4*>(static_cast<float*>(a.y) + o);
-        if constexpr (OUT == kOutF32Acc) {
-          const f32x4 old = *dst;
-          v = f32x4{old[0] + v[0], old[1] + v[1], old[2] + v[2], old[3] + v[3]};
-        }
-        *dst = v;
+      put_out<BLOCK, OUT>(a, m, n, acc[i][j]);
+    }
+  }
+}
+
+// The smaller tiles: WN x WM waves of NI x NJ MFMA tiles each (a tile of TN = 16 NI WN weight rows x TM = 16 NJ WM
+// tokens), for products whose 256 x 256 tiles would leave CUs without work. The arithmetic of an output is the same (its
+// K blocks in order, each folded once), so which tile a shape gets changes no bit of an unsplit result.
+//
+// What bounds these is the way of the operands to the CU, not the MFMAs: with the loads to LDS taken out (and wrong
+// results) 200 x 7168 x 5120 in 128 x 64 tiles takes 13.8 us instead of 21.1, without MFMAs 21.1, without the LDS reads
+// 20.8. So the K loop is built around loads in flight: S stages of direct loads to LDS, of which S - 1 are on their way
+// while one is multiplied. The fragments of block kb + 1 are read from LDS while block kb is multiplied (two register
+// sets), spread with the loads over the block's weight tiles: issued in one burst ahead of the MFMAs they delayed them
+// (26.5 us at 512 x 5120 x 5120 in 128 x 128 tiles, 32.6 with the bursts).
+template <int NI, int NJ, int WN, int WM>
+struct TileShape {
+  static constexpr int kTN = 16 * NI * WN, kTM = 16 * NJ * WM, kNW = WN * WM;
+  static constexpr int kLW = kTN * 8 / (64 * kNW), kLX = kTM * 8 / (64 * kNW);  // 16-byte loads per lane and stage
+  static constexpr int kScale = (kTM > 64 * kNW ? kTM / 64 : kNW) * 256;  // a 256-byte run per wave
+  static constexpr int kStageB = (kTN + kTM) * kRowBytes + kScale;
+  static_assert(kLW * 64 * kNW == kTN * 8 && kLX * 64 * kNW == kTM * 8, "whole loads per wave");
+  static_assert(128 % (16 * NI) == 0, "a wave's weight rows lie in one scale block");
+};
+
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+  static_assert(N < 64, "vmcnt holds at most 63");
+  __builtin_amdgcn_s_waitcnt(0x0f70 | (N & 15) | ((N >> 4) << 14));
+}
+
+template <bool BLOCK, int OUT, int NI, int NJ, int WN, int WM, int S>
+__global__ void __launch_bounds__(64 * WN * WM) prefill_tile_kernel(const PrefillArgs a) {
+  using Sh = TileShape<NI, NJ, WN, WM>;
+  constexpr int TN = Sh::kTN, TM = Sh::kTM, NW = Sh::kNW, LW = Sh::kLW, LX = Sh::kLX, STG = Sh::kStageB;
+  constexpr int kVm = LW + LX + (BLOCK ? 1 : 0);  // loads per lane and stage (the scales': waves past TM tokens load none)
+  static_assert(TM <= 64 * NW, "one scale per lane");
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 15, t = lane >> 4;
+  const int wn = wave % WN, wm = wave / WN;
+
+  // Tile order: XCD b % 8 takes a contiguous range of the tiles; groups of kGroupN weight tiles x every token tile,
+  // weight tiles fastest, so that a weight tile's readers run on one XCD, a little after one another.
+  const int nb = gridDim.x, b = blockIdx.x, x = b & 7;
+  const int tile = x * (nb >> 3) + min(x, nb & 7) + (b >> 3);
+  const int grp = tile / (kGroupN * a.tiles_m), rem = tile % (kGroupN * a.tiles_m);
+  const int gsize = min(kGroupN, a.tiles_n - grp * kGroupN);
+  const int tn = grp * kGroupN + rem % gsize, tm = rem / gsize;
+  const int n0 = tn * TN, m0 = tm * TM;
+
+  const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(a.w), 0, a.N * a.K, 0x00020000);
+  const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(a.xq), 0, a.M * a.K, 0x00020000);
+  const __amdgpu_buffer_rsrc_t sr =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.xs), 0, a.M * a.KB * 4, 0x00020000);
+
+  // Load-to-LDS plan as in prefill_fp8_kernel: load i of wave w fills 8 rows from (i * NW + w) * 8. A row past the
+  // operand gets an offset that is out of range by itself.
+  constexpr unsigned kOob = 0x80000000u;
+  unsigned wsrc[LW], xsrc[LX], ssrc = kOob;
+#pragma unroll
+  for (int i = 0; i < LW; ++i) {
+    const int row = (i * NW + wave) * 8 + (lane >> 3), u = (lane & 7) ^ swz(row), n = n0 + row;
+    wsrc[i] = n < a.N ? static_cast<unsigned>((n >> 4) * a.KB * kTileBytesFp8 +
+                                              (((((row & 15) >> 3) * 2 + (u & 1)) * 8 + (row & 7)) * 4 + (u >> 1)) * 16)
+                      : kOob;
+  }
+#pragma unroll
+  for (int i = 0; i < LX; ++i) {
+    const int row = (i * NW + wave) * 8 + (lane >> 3), u = (lane & 7) ^ swz(row), m = m0 + row;
+    xsrc[i] = m < a.M ? static_cast<unsigned>(m * a.K + u * 16) : kOob;
+  }
+  if constexpr (BLOCK) {
+    const int row = wave * 64 + lane;
+    if (row < TM && m0 + row < a.M) ssrc = static_cast<unsigned>((m0 + row) * a.KB * 4);
+  }
+  // Loads [v0, v1) of a stage's kVm. (A block past the end is issued out of range: every wait count then holds on
+  // every path.)
+  auto issue_some = [&](int st, int kb, int v0, int v1) {
+    const unsigned oob = kb < a.KB ? 0u : kOob;
+    uint8_t* base = smem + st * STG;
+#pragma unroll
+    for (int v = v0; v < v1; ++v) {
+      if (v < LW) dma16(wr, base + (v * NW + wave) * 1024, wsrc[v] | oob, kb * kTileBytesFp8);
+      else if (v < LW + LX)
+        dma16(xr, base + TN * kRowBytes + ((v - LW) * NW + wave) * 1024, xsrc[v - LW] | oob, kb * kRowBytes);
+      else dma4(sr, base + (TN + TM) * kRowBytes + wave * 256, ssrc | oob, kb * 4);
+    }
+  };
+  // all loads but those of the newest KEEP stages have landed
+  auto wait_stages = [&](auto keep) {
+    wait_vm<decltype(keep)::value * kVm>();
+  };
+
+  f32x4 acc[NI][NJ];
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  const int nrow = n0 + wn * NI * 16;
+  const float* wsrow = BLOCK ? a.ws + static_cast<size_t>(min(nrow, a.N - 1) >> 7) * a.KB : nullptr;
+  struct Frags {
+    i32x8 a[NI], b[NJ];
+    float xs[NJ], ws;
+  };
+  // share i of NI of a block's fragment reads
+  auto read_some = [&](Frags& f, int st, int kb, int i) {
+    const uint8_t* sa = smem + st * STG;
+    if constexpr (BLOCK) {
+      if (i == 0) {
+        const float* sxs = reinterpret_cast<const float*>(sa + (TN + TM) * kRowBytes);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) f.xs[j] = sxs[wm * NJ * 16 + 16 * j + r];
+        f.ws = scalar_load(wsrow + min(kb, a.KB - 1));
       }
+    }
+    f.a[i] = fragment(sa, wn * NI * 16 + 16 * i + r, t);
+#pragma unroll
+    for (int j = i * NJ / NI; j < (i + 1) * NJ / NI; ++j) f.b[j] = fragment(sa + TN * kRowBytes, wm * NJ * 16 + 16 * j + r, t);
+  };
+
+#pragma unroll
+  for (int s = 0; s < S; ++s) issue_some(s, s, 0, kVm);
+  Frags f0, f1;
+  wait_stages(std::integral_constant<int, S - 1>{});
+  __builtin_amdgcn_s_barrier();
+#pragma unroll
+  for (int i = 0; i < NI; ++i) read_some(f0, 0, 0, i);
+  // A block's products, one weight tile at a time; before(i) is issued ahead of tile i's MFMAs and tile i - 1's fold
+  // behind them.
+  auto multiply = [&](const Frags& cur, auto&& before) {
+    float sc[NJ];
+    f32x4 pr[2][NJ];
+    if constexpr (BLOCK) {
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) sc[j] = cur.xs[j] * cur.ws;
+    }
+    auto fold = [&](int i) {
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) acc[i][j][v] = __builtin_fmaf(pr[i & 1][j][v], sc[j], acc[i][j][v]);
+    };
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      before(i);
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        if constexpr (BLOCK)
+          pr[i & 1][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(cur.a[i], cur.b[j], f32x4{0.f, 0.f, 0.f, 0.f}, 0,
+                                                                          0, 0, 0, 0, 0);
+        else
+          acc[i][j] =
+              __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(cur.a[i], cur.b[j], acc[i][j], 0, 0, 0, 0, 0, 0);
+      }
+      if (BLOCK && i > 0) fold(i - 1);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (BLOCK) fold(NI - 1);
+  };
+  int st = 0;
+  auto step = [&](Frags& cur, Frags& nxt, int kb) {
+    const int st1 = st + 1 == S ? 0 : st + 1;
+    // block kb + 1 has landed, and this wave has read its fragments of block kb; past the barrier every wave has,
+    // so stage st takes block kb + S (the empty statements keep the reads on their side of the barrier)
+    asm volatile("" ::: "memory");
+    wait_stages(std::integral_constant<int, S - 2>{});
+    LQ_WAIT_LGKM0();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    multiply(cur, [&](int i) {
+      read_some(nxt, st1, kb + 1, i);
+      issue_some(st, kb + S, i * kVm / NI, (i + 1) * kVm / NI);
+    });
+    st = st1;
+  };
+  // (two whole steps per round, the odd block after them: a branch between a block's instructions would part them)
+  int kb = 0;
+  for (; kb + 2 <= a.KB; kb += 2) {
+    step(f0, f1, kb);
+    step(f1, f0, kb + 1);
+  }
+  if (kb < a.KB) multiply(f0, [](int) {});
+  LQ_WAIT_VM0();  // no load to LDS outlives the workgroup
+
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) {
+    const int m = m0 + wm * NJ * 16 + 16 * j + r;
+    if (m >= a.M) continue;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int n = nrow + 16 * i + 4 * t;
+      if (n < a.N) put_out<BLOCK, OUT>(a, m, n, acc[i][j]);
     }
   }
 }
@@ -401,6 +610,56 @@ __global__ void __launch_bounds__(256) quant_fp8_pt_kernel(const void* __restric
   }
 }
 
+template <bool BLOCK, int OUT, int NI, int NJ, int WN, int WM, int S>
+int tile_launch(PrefillArgs a, const char* name, hipStream_t s) {
+  using Sh = TileShape<NI, NJ, WN, WM>;
+  a.tiles_m = cdiv(a.M, Sh::kTM);
+  a.tiles_n = cdiv(a.N, Sh::kTN);
+  constexpr int lds = S * Sh::kStageB;
+  static_assert(lds <= 160 * 1024, "LDS of a CU");
+  static const hipError_t attr =
+      hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_tile_kernel<BLOCK, OUT, NI, NJ, WN, WM, S>),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  if (attr != hipSuccess) return fail(LQ_ERR_LAUNCH, std::string(name) + ": " + hipGetErrorString(attr));
+  hipLaunchKernelGGL((prefill_tile_kernel<BLOCK, OUT, NI, NJ, WN, WM, S>),
+                     dim3(static_cast<unsigned>(a.tiles_m) * static_cast<unsigned>(a.tiles_n)), dim3(64 * WN * WM), lds, s, a);
+  return check_launch(name);
+}
+
+// The tile of a product, by an estimate of its time. `single` is what a K block of a tile costs on a CU that has one
+// (microseconds, weights from memory), `pair` what one of two resident tiles' costs together; the larger the tile, the
+// less each output costs, but tiles come in whole numbers per CU, so a product with few of them is done sooner in
+// smaller ones. A launch costs 4 us; a split last round of 256 x 256 tiles 10 us more and 0.07 us per part, for the
+// exchange. The smallest sum wins, the 256 x 256 tile unless another is 5 % better. Measured, block-scaled (M x N x K,
+// us, rotating over 600 MB of weights): 100 x 5120 x 5120 35 -> 15 (64 x 64), 200 x 7168 x 5120 40 -> 21 (128 x 64),
+// 300 x 5120 x 17408 86 -> 70 (128 x 64), 512 x 5120 x 5120 42 -> 31 (128 x 128), 500 x 17408 x 5120 83 -> 80
+// (128 x 128 x2); 1000 x 5120 x 17408 stays at 110 (132 in 128 x 128 x2). 64 x 128 (15 % faster at 300 x 5120 x 17408,
+// 10 % slower elsewhere) and 128 x 256 (7 % faster at 777 x 5120 x 6144, 9 % slower at 256 x 17408 x 5120) were not
+// worth their kernels.
+enum PrefillTile { kT256x256, kT64x64, kT128x64, kT128x128, kT128x128x2 };  // x2: two stages, two tiles per CU
+PrefillTile choose_tile(const PrefillArgs& a, long long cus) {
+  constexpr double kLaunch = 4., kSplit = 10., kPart = 0.07, kBig = 1.72;
+  double best = kLaunch + a.KB * kBig * static_cast<double>((a.full + cus - 1) / cus);
+  if (a.rem) best += kBig * a.KB / a.S + kSplit + kPart * a.rem * a.S;
+  best *= 0.95;
+  PrefillTile tile = kT256x256;
+  struct Kind {
+    PrefillTile tile;
+    int tn, tm;
+    double single, pair;
+  };
+  for (const Kind& k : {Kind{kT64x64, 64, 64, 0.275, 0.52}, Kind{kT128x64, 128, 64, 0.44, 0.74},
+                        Kind{kT128x128, 128, 128, 0.65, 1.3}, Kind{kT128x128x2, 128, 128, 0.85, 1.02}}) {
+    const long long n = (static_cast<long long>(cdiv(a.N, k.tn)) * cdiv(a.M, k.tm) + cus - 1) / cus;
+    const double us = kLaunch + a.KB * (static_cast<double>(n / 2) * k.pair + static_cast<double>(n % 2) * k.single);
+    if (us < best) {
+      best = us;
+      tile = k.tile;
+    }
+  }
+  return tile;
+}
+
 template <bool BLOCK, int OUT>
 int prefill_launch(PrefillArgs a, const char* name, hipStream_t s) {
   const std::string nm(name);
@@ -432,6 +691,13 @@ int prefill_launch(PrefillArgs a, const char* name, hipStream_t s) {
     a.rem = 0;
   }
   a.full = static_cast<int>(tiles - a.rem);
+  switch (choose_tile(a, P)) {
+    case kT64x64: return tile_launch<BLOCK, OUT, 2, 2, 2, 2, 4>(a, name, s);
+    case kT128x64: return tile_launch<BLOCK, OUT, 4, 2, 2, 2, 3>(a, name, s);
+    case kT128x128: return tile_launch<BLOCK, OUT, 4, 4, 2, 2, 4>(a, name, s);
+    case kT128x128x2: return tile_launch<BLOCK, OUT, 4, 4, 2, 2, 2>(a, name, s);
+    default: break;
+  }
   const long long blocks = a.full + (a.rem ? 8LL * cdiv(a.rem, 8) * a.S : 0);
   if (a.rem) {
     // rem * S <= P partial tiles: the bound is reserved once per device (lq_init, or here on first use) and never

@@ -79,6 +79,22 @@ def test_prefill_small_full(L, M, N, K):
     assert np.array_equal(bf16_host(y), bf16_host(y2))
 
 
+# one shape for each of the smaller tiles (64 x 64, 128 x 64, 128 x 128 with four and with two stages), with a last
+# token tile of a few rows and fewer, as many and more K blocks than the tile has stages, odd counts among them
+@pytest.mark.parametrize("M,N", [(81, 384), (257, 4224), (513, 4224), (1026, 4224)])
+@pytest.mark.parametrize("K", [128, 384, 640])
+def test_prefill_small_tiles(L, M, N, K):
+    wq, ws, xq, xs, tw = prefill_case(L, M, N, K, 60 + M)
+    y = L.prefill_fp8_block(to_dev(xq), to_dev(xs), tw, to_dev(ws), N)
+    rows = np.unique(np.r_[0, 15, 16, 63, 64, M // 2, M - 2, M - 1])
+    check(bf16_host(y)[rows], O.prefill_fp8_rows(xq, xs, rows, wq, ws), f"block M={M} N={N} K={K}")
+    # the same K blocks in the same order whatever the tile: a row of a larger call is bit for bit the smaller call's
+    sub = L.prefill_fp8_block(to_dev(xq[:17]), to_dev(xs[:17]), tw, to_dev(ws), N)
+    assert np.array_equal(bf16_host(sub), bf16_host(y)[:17])
+    yt = L.prefill_gemm_fp8(to_dev(xq), tw, 3.0e-4, N)
+    check_f32(yt.cpu().numpy()[rows].astype(np.float64), pt_ref(xq, wq, 3.0e-4, rows), f"per-tensor M={M} N={N} K={K}")
+
+
 def test_prefill_stray_columns_and_rows(L):
     M, N, K = 70, 256, 256
     wq, ws, xq, xs, tw = prefill_case(L, M, N, K, 7)
