@@ -11,31 +11,36 @@
 // significant bits and lies in [2^-10, 2688] - and multiplied on v_mfma_f32_16x16x32_f16 with FP32
 // accumulation across all of K; alpha is applied at the end.
 //
-//  * A workgroup (8 waves: 2 along the weights x 4 along the tokens) computes 256 weight rows x 256 tokens; each
-//    wave 128 x 64 (8 x 4 MFMA tiles). Per 128-value chunk a lane holds the raw 16 bytes (32 E2M1 values) and
-//    2 scale bytes of its row for each of its 8 weight tiles and 4 token tiles, and dequantizes one 8-value
-//    step at a time: lane (r, t) supplies K 32t + 8s .. +8 at step s for both operands (a permutation of K
-//    inside the chunk, harmless as both operands use it; the weights' tiled layout holds exactly these 16
-//    bytes per (row, t), slot r * 4 + t).
-//  * Operands go from global memory straight to LDS (buffer loads with the LDS flag): per chunk 16 KB of
-//    weight values, 2 KB of weight scales, and the same for the activations, in three stages (108 KB), so the
-//    loads of chunk c + 2 overlap the compute of chunk c. The 16-byte units of a 64-byte row are XOR-swizzled
-//    by swz4(row) so the 16-byte fragment reads are conflict free whether the LDS serves 8 or 16 lanes of
-//    them per cycle.
+//  * A wave computes 128 weight rows x 64 tokens (8 x 4 MFMA tiles, 128 accumulator registers; SwiGLU: 64 gate rows and
+//    the same 64 up rows). Per 128-value chunk a lane holds the raw 16 bytes (32 E2M1 values) and the 2 scales of its
+//    row for each of its 8 weight tiles and 4 token tiles, and dequantizes one 8-value step at a time: lane (r, t)
+//    supplies K 32t + 8s .. +8 at step s for both operands (a permutation of K inside the chunk, harmless as both
+//    operands use it; the weights' tiled layout holds exactly these 16 bytes per (row, t), slot r * 4 + t).
+//  * The 8 waves of a workgroup are WM along the tokens x WK = 8 / WM along K, so a tile is 64 WM tokens high and a prompt
+//    of a few hundred tokens still gives every CU two waves per SIMD, at the wave tile's ratio of dequantization to
+//    MFMAs. Wave k of a K group takes chunks k, k + WK, ..; the group's FP32 sums meet in LDS at the end and are added
+//    in wave order.
+//  * Nothing is shared while a wave computes, so there are no barriers: each wave streams its own operands to its own
+//    13.5 KB of LDS by direct loads, takes a landed chunk into registers (60 of them) and at once has the next one loaded
+//    over it, which then has the whole chunk's 128 MFMAs to arrive.
+//  * LDS of a wave: [weight values 128 x 64 B][weight scales 128 x 8][token values 64 x 64][token scales 64 x 8]. The
+//    16-byte units of a 64-byte row are XOR-swizzled by swz4(row) so the 16-byte fragment reads are conflict free whether
+//    the LDS serves 8 or 16 lanes of them per cycle; four lanes of a load read one run of 64 bytes.
+//
+// What bounds it: the dequantization and the MFMAs share the SIMD's issue (3 VALU instructions per MFMA). Tiles of 256 x
+// 256 over 8 waves, which read a step's word from LDS just ahead of its use, took 430 us at 300 x 5120 x 17408 (40 tiles
+// on 256 CUs), 447 at 2048 x 5120 x 17408 and 760 for SwiGLU at 2048 x 17408 x 5120: now 67, 321 and 637.
 #include "lq_common.hpp"
 
-#include <algorithm>
 #include <string>
 
 namespace lq {
 namespace {
 
-constexpr int kBN = 256, kBM = 256, kThreads = 512, kStages = 3, kGroupN = 4;
-constexpr int kValBytes = 256 * 64;     // one operand's chunk of values in LDS
-constexpr int kScBytes = 256 * 8;       // its E4M3 scales
-constexpr int kStage = 2 * (kValBytes + kScBytes);
-// stage layout: [A values][A scales][B values][B scales]
-constexpr int kOffAs = kValBytes, kOffB = kValBytes + kScBytes, kOffBs = 2 * kValBytes + kScBytes;
+constexpr int kThreads = 512;
+constexpr int kWaveOffX = 128 * 72, kWaveStage = kWaveOffX + 64 * 72;  // a wave's LDS: weights, then tokens
+constexpr int kRedWave = 16 * 1024;  // a wave's sums of four weight tiles x four token tiles
+static_assert(kRedWave >= kWaveStage, "the reduction takes the larger part of LDS");
 
 // 16 lanes read one 16-byte unit each of rows r .. r + 15 (r % 16 == 0): banks (row % 4, unit) must be distinct
 // over the 16 rows, and (row % 2, unit) over each aligned 8.
@@ -56,7 +61,7 @@ struct Nvfp4Args {
   float gscale_out;  // SwiGLU: 1 / out_input_scale
   uint8_t* q_out;    // [M][N/2]
   uint8_t* sf_out;   // [M][N/16]
-  int tiles_m, tiles_n, rows_per_tile;  // rows_per_tile: 256 (plain) or 128 output columns (SwiGLU)
+  int tiles_m, tiles_n;
 };
 
 typedef __attribute__((address_space(3))) void* lds_ptr;
@@ -69,11 +74,13 @@ __device__ __forceinline__ void dma4(__amdgpu_buffer_rsrc_t rs, uint8_t* lds, in
   __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr)(lds), 4, voff, __builtin_amdgcn_readfirstlane(soff), 0, 0);
 }
 
-// Step s of a lane's raw chunk (word d = 8 E2M1 codes of its 16 bytes, two E4M3 scale bytes): 8 FP16 values
-// e2m1 * scale (exact); steps 0, 1 use the first scale (K 32t .. +16), steps 2, 3 the second.
-__device__ __forceinline__ u32x4 deq_word(uint32_t d, uint32_t sc, int s) {
-  const uint32_t b = (s < 2) ? (sc & 0xffu) : ((sc >> 8) & 0xffu);
-  const f16x2 scv = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(b | (b << 8), 1.0f, false);
+// A lane's two E4M3 block scales of a chunk as FP16 (exact): one conversion per row and chunk.
+__device__ __forceinline__ f16x2 scale_pair(uint32_t sc) { return __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(sc, 1.0f, false); }
+
+// Step s of a lane's raw chunk (word d = 8 E2M1 codes of its 16 bytes, its scale pair): 8 FP16 values e2m1 * scale
+// (exact); steps 0, 1 use the first scale (K 32t .. +16), steps 2, 3 the second.
+__device__ __forceinline__ u32x4 deq_word(uint32_t d, f16x2 sc, int s) {
+  const f16x2 scv = f16x2{sc[s >> 1], sc[s >> 1]};
   const f16x2 e0 = fp4x2_to_f16x2<0>(d) * scv, e1 = fp4x2_to_f16x2<1>(d) * scv;
   const f16x2 e2 = fp4x2_to_f16x2<2>(d) * scv, e3 = fp4x2_to_f16x2<3>(d) * scv;
   return u32x4{__builtin_bit_cast(uint32_t, e0), __builtin_bit_cast(uint32_t, e1), __builtin_bit_cast(uint32_t, e2),
@@ -82,75 +89,104 @@ __device__ __forceinline__ u32x4 deq_word(uint32_t d, uint32_t sc, int s) {
 
 #define LQ_WAIT_VM(n) asm volatile("s_waitcnt vmcnt(" #n ")" ::: "memory")
 
-template <bool SWIGLU>
+// Four outputs of one token, columns n .. n + 3.
+__device__ __forceinline__ void put_out(const Nvfp4Args& a, int m, int n, f32x4 acc) {
+  f32x4 v = f32x4{acc[0] * a.alpha, acc[1] * a.alpha, acc[2] * a.alpha, acc[3] * a.alpha};
+  f32x4* dst = reinterpret_cast<f32x4*>(a.y + static_cast<size_t>(m) * a.ldy + n);
+  if (a.accumulate) {
+    const f32x4 o = *dst;
+    v = f32x4{o[0] + v[0], o[1] + v[1], o[2] + v[2], o[3] + v[3]};
+  }
+  *dst = v;
+}
+
+// SwiGLU: the lane's four values of the 16-column output block from column ncol, token m (every lane of the wave calls
+// it: a block's values are in lanes r, r + 16, r + 32, r + 48). up: alpha_up already applied.
+__device__ __forceinline__ void put_swiglu(const Nvfp4Args& a, int m, int ncol, int t, f32x4 gate, f32x4 up) {
+  float v[4], amax = 0.f;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float gv = gate[e] * a.alpha;
+    v[e] = bf16_to_f32(f32_to_bf16((gv / (1.f + __expf(-gv))) * up[e]));
+    amax = fmaxf(amax, fabsf(v[e]));
+  }
+  amax = fmaxf(amax, __shfl_xor(amax, 16));
+  amax = fmaxf(amax, __shfl_xor(amax, 32));
+  const float sraw = a.gscale_out * (amax * (1.f / 6.f));
+  const uint32_t sc = __builtin_amdgcn_cvt_pk_fp8_f32(fminf(sraw, 448.f), 0.f, 0, false) & 0xffu;
+  const float sv = e4m3_to_f32(sc);
+  const float os = sv != 0.f ? 1.f / (sv * (1.f / a.gscale_out)) : 0.f;
+  if (m < a.M && ncol < a.N) {
+    uint8_t* qr = a.q_out + static_cast<size_t>(m) * (a.N / 2) + ncol / 2 + 2 * t;
+    const uint32_t b0 = e2m1x2_rne(v[0] * os, v[1] * os);
+    const uint32_t b1 = e2m1x2_rne(v[2] * os, v[3] * os);
+    *reinterpret_cast<uint16_t*>(qr) = static_cast<uint16_t>(b0 | (b1 << 8));
+    if (t == 0) a.sf_out[static_cast<size_t>(m) * (a.N / 16) + ncol / 16] = static_cast<uint8_t>(sc);
+  }
+}
+
+template <bool SWIGLU, int WM>
 __global__ void __launch_bounds__(kThreads) prefill_nvfp4_kernel(const Nvfp4Args a) {
+  constexpr int WK = 8 / WM, TN = SWIGLU ? 64 : 128, TM = 64 * WM;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, t = lane >> 4;
-  const int wn = wave & 1, wm = wave >> 1;
+  const int wk = wave % WK, wm = wave / WK;
 
-  // grouped raster per XCD, as the FP8 prefill kernel
-  const int nb = gridDim.x, b = blockIdx.x;
-  int tile = b;
-  if ((nb & 7) == 0) tile = (b & 7) * (nb >> 3) + (b >> 3);
-  const int grp = tile / (kGroupN * a.tiles_m), rem = tile % (kGroupN * a.tiles_m);
-  const int gsize = min(kGroupN, a.tiles_n - grp * kGroupN);
-  const int tn = grp * kGroupN + rem % gsize, tm = rem / gsize;
-  const int n0 = tn * a.rows_per_tile, m0 = tm * kBM;
+  // Tile order: XCD b % 8 takes a contiguous range of the tiles; groups of 8 weight tiles x every token tile, weight
+  // tiles fastest.
+  constexpr int kGroup = 8;
+  const int nb = gridDim.x, b = blockIdx.x, x = b & 7;
+  const int tile = x * (nb >> 3) + min(x, nb & 7) + (b >> 3);
+  const int grp = tile / (kGroup * a.tiles_m), rem = tile % (kGroup * a.tiles_m);
+  const int gsize = min(kGroup, a.tiles_n - grp * kGroup);
+  const int n0 = (grp * kGroup + rem % gsize) * TN, m0 = (rem / gsize) * TM + wm * 64;
 
-  // weight LDS rows: plain, row = n - n0 (256 rows of w); SwiGLU, rows 0..127 = gate rows n0 .., 128..255 = up
-  const int rows_w = SWIGLU ? a.N : a.N;
   const int blkb = a.wsf ? kValueBytesFp4 : kTileBytesFp4;
-  const int nbytes = (rows_w / 16) * a.C * blkb;
-  const __amdgpu_buffer_rsrc_t wr1 = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(a.w), 0, nbytes, 0x00020000);
-  const __amdgpu_buffer_rsrc_t wr2 = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(SWIGLU ? a.w2 : a.w), 0,
-                                                                        nbytes, 0x00020000);
-  const int sbytes = a.wsf ? (rows_w / 16) * a.C * 128 : nbytes;
-  const __amdgpu_buffer_rsrc_t sr1 = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint8_t*>(a.wsf ? a.wsf : a.w), 0, sbytes, 0x00020000);
-  const __amdgpu_buffer_rsrc_t sr2 = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint8_t*>(SWIGLU ? (a.wsf2 ? a.wsf2 : a.w2) : (a.wsf ? a.wsf : a.w)), 0, sbytes, 0x00020000);
-  const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(a.xq), 0, a.M * (a.K / 2), 0x00020000);
-  const __amdgpu_buffer_rsrc_t xsr = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(a.xs), 0, a.M * (a.K / 16), 0x00020000);
-
-  // Load plan. Values: load i (0, 1) of wave w writes LDS units P = (i * 8 + w) * 64 + lane: row (i * 8 + w) * 16 +
-  // lane / 4, physical unit lane % 4, source unit u = lane % 4 ^ swz4(row) (row % 16 = lane / 4: the same for
-  // both loads). Scales: thread x writes 4 bytes at 4x: row x / 2, half x % 2.
-  const int vrow = wave * 16 + (lane >> 2), vu = (lane & 3) ^ swz4(lane >> 2);
-  auto wrow_src = [&](int row) {  // (matrix half, weight row) of LDS row `row`
-    return SWIGLU ? (n0 + (row & 127)) : (n0 + row);
+  const int nbytes = (a.N / 16) * a.C * blkb, sbytes = a.wsf ? (a.N / 16) * a.C * 128 : nbytes;
+  auto rsrc = [](const uint8_t* p, int bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(p), 0, bytes, 0x00020000);
   };
-  int wsrc[2], wssrc;
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int row = i * 128 + vrow, n = wrow_src(row);
-    const int slot = (n & 15) * 4 + vu;
-    wsrc[i] = n < a.N ? ((n >> 4) * a.C) * blkb + slot * 16 : static_cast<int>(0x80000000u);
-  }
-  const int srow = static_cast<int>(threadIdx.x) >> 1, shalf = threadIdx.x & 1;
-  {
-    const int n = wrow_src(srow);
-    const int so = a.wsf ? ((n >> 4) * a.C) * 128 + (n & 15) * 8 : ((n >> 4) * a.C) * blkb + 1024 + (n & 15) * 8;
-    wssrc = n < a.N ? so + shalf * 4 : static_cast<int>(0x80000000u);
-  }
-  const int sstep = a.wsf ? 128 : blkb;  // scale bytes per chunk step of a block
-  int xsrc[2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int m = m0 + i * 128 + vrow;
-    xsrc[i] = m < a.M ? m * (a.K / 2) + vu * 16 : static_cast<int>(0x80000000u);
-  }
-  const int xssrc = (m0 + srow) < a.M ? (m0 + srow) * (a.K / 16) + shalf * 4 : static_cast<int>(0x80000000u);
+  const __amdgpu_buffer_rsrc_t wr1 = rsrc(a.w, nbytes), wr2 = rsrc(SWIGLU ? a.w2 : a.w, nbytes);
+  const __amdgpu_buffer_rsrc_t sr1 = rsrc(a.wsf ? a.wsf : a.w, sbytes);
+  const __amdgpu_buffer_rsrc_t sr2 = rsrc(SWIGLU ? (a.wsf2 ? a.wsf2 : a.w2) : (a.wsf ? a.wsf : a.w), sbytes);
+  const __amdgpu_buffer_rsrc_t xr = rsrc(a.xq, a.M * (a.K / 2)), xsr = rsrc(a.xs, a.M * (a.K / 16));
 
-  auto issue = [&](int st, int c) {
-    uint8_t* base = smem + st * kStage;
-    dma16(wr1, base + (0 * 8 + wave) * 1024, wsrc[0], c * blkb);
-    dma16(wr2, base + (1 * 8 + wave) * 1024, wsrc[1], c * blkb);
-    if (SWIGLU ? wave < 4 : true) dma4(sr1, base + kOffAs + wave * 256, wssrc, c * sstep);
-    else dma4(sr2, base + kOffAs + wave * 256, wssrc, c * sstep);
-    dma16(xr, base + kOffB + (0 * 8 + wave) * 1024, xsrc[0], c * 64);
-    dma16(xr, base + kOffB + (1 * 8 + wave) * 1024, xsrc[1], c * 64);
-    dma4(xsr, base + kOffBs + wave * 256, xssrc, c * 8);
+  // Weight rows are whole tiles of a matrix with N % 128 == 0: always in range. Weight tile i (0 .. 7) of the wave is
+  // 16-row tile n0 / 16 + i (SwiGLU: + i % 4, the up matrix from i = 4); a lane loads unit lane % 4 of row lane / 4 of a
+  // tile's values, 4 bytes of two tiles' scales.
+  const int srow = lane >> 2, su = (lane & 3) ^ swz4(srow);
+  const int wsrc = srow * 64 + su * 16, tstep = a.C * blkb, wbase = (n0 >> 4) * tstep;
+  const int sblk = a.wsf ? 128 : blkb, sstep = a.C * sblk;
+  const int ssrc = (lane >> 5) * sstep + (a.wsf ? 0 : 1024) + (lane & 31) * 4, sbase = (n0 >> 4) * sstep;
+  constexpr unsigned kOob = 0x80000000u;
+  unsigned xsrc[4], xssrc[2];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int m = m0 + 16 * j + srow;
+    xsrc[j] = m < a.M ? static_cast<unsigned>(m * (a.K / 2) + su * 16) : kOob;
+  }
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int m = m0 + 32 * j + (lane >> 1);
+    xssrc[j] = m < a.M ? static_cast<unsigned>(m * (a.K / 16) + (lane & 1) * 4) : kOob;
+  }
+  uint8_t* lds = smem + wave * kWaveStage;
+  // load v of a chunk's 18
+  constexpr int kLoads = 18;
+  auto issue_one = [&](int c, int v) {
+    if (v < 8) {
+      if (SWIGLU && v >= 4) dma16(wr2, lds + v * 1024, wsrc, wbase + (v - 4) * tstep + c * blkb);
+      else dma16(wr1, lds + v * 1024, wsrc, wbase + v * tstep + c * blkb);
+    } else if (v < 12) {
+      const int p = v - 8;
+      if (SWIGLU && p >= 2) dma4(sr2, lds + 128 * 64 + p * 256, ssrc, sbase + 2 * (p - 2) * sstep + c * sblk);
+      else dma4(sr1, lds + 128 * 64 + p * 256, ssrc, sbase + 2 * p * sstep + c * sblk);
+    } else if (v < 16) {
+      dma16(xr, lds + kWaveOffX + (v - 12) * 1024, xsrc[v - 12], c * 64);
+    } else {
+      dma4(xsr, lds + kWaveOffX + 64 * 64 + (v - 16) * 256, xssrc[v - 16], c * 8);
+    }
   };
 
   f32x4 acc[8][4];
@@ -159,117 +195,115 @@ __global__ void __launch_bounds__(kThreads) prefill_nvfp4_kernel(const Nvfp4Args
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  issue(0, 0);
-  if (a.C > 1) issue(1, 1);
-  else issue(1, 0);  // keeps the wait counts uniform; the stage is never read
-  LQ_WAIT_VM(6);
-  __builtin_amdgcn_s_barrier();
-  for (int c = 0; c < a.C; ++c) {
-    const int st = c % kStages;
-    const uint8_t* sa = smem + st * kStage;
-    // loads of chunk c + 2 (a repeat of the last chunk past the end, never read, keeps the waits uniform)
-    issue((c + 2) % kStages, min(c + 2, a.C - 1));
-    // the scale bytes are held for the chunk; each tile's word of step s is read when needed
-    uint32_t as[8], bs[4];
+  const int last = a.C - 1;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) as[i] = *reinterpret_cast<const uint16_t*>(sa + kOffAs + (wn * 128 + 16 * i + r) * 8 + t * 2);
+  for (int v = 0; v < kLoads; ++v) issue_one(min(wk, last), v);
+  for (int c = wk; c < a.C; c += WK) {
+    LQ_WAIT_VM(0);
+    u32x4 aw[8], bw[4];
+    f16x2 as[8], bs[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) bs[j] = *reinterpret_cast<const uint16_t*>(sa + kOffBs + (wm * 64 + 16 * j + r) * 8 + t * 2);
+    for (int j = 0; j < 4; ++j) {
+      bw[j] = *reinterpret_cast<const u32x4*>(lds + kWaveOffX + val_off(16 * j + r, t));
+      bs[j] = scale_pair(*reinterpret_cast<const uint16_t*>(lds + kWaveOffX + 64 * 64 + (16 * j + r) * 8 + t * 2));
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      aw[i] = *reinterpret_cast<const u32x4*>(lds + val_off(16 * i + r, t));
+      as[i] = scale_pair(*reinterpret_cast<const uint16_t*>(lds + 128 * 64 + (16 * i + r) * 8 + t * 2));
+    }
+    // every read has returned before the next chunk's loads go over them (past the end the last chunk again, never read)
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    const int next = min(c + WK, last);
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
       u32x4 bf[4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-        bf[j] = deq_word(*reinterpret_cast<const uint32_t*>(sa + kOffB + val_off(wm * 64 + 16 * j + r, t) + 4 * s), bs[j], s);
+      for (int j = 0; j < 4; ++j) bf[j] = deq_word(bw[j][s], bs[j], s);
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        // (empty volatile statements keep each read in its place: hoisted, the reads run the wave out of registers)
-        asm volatile("" ::: "memory");
-        const uint32_t d = *reinterpret_cast<const uint32_t*>(sa + val_off(wn * 128 + 16 * i + r, t) + 4 * s);
-        const u32x4 af = deq_word(d, as[i], s);
+        // (one or two of the loads per weight tile: a burst would hold the wave up)
+        if (s * 8 + i < kLoads) issue_one(next, s * 8 + i);
+        const u32x4 af = deq_word(aw[i][s], as[i], s);
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc[i][j] = mfma16x16x32(af, bf[j], acc[i][j], true);
       }
-      asm volatile("" ::: "memory");
     }
-    // this thread's loads of chunk c + 1 have landed (only chunk c + 2's six are newer); after the barrier every
-    // wave's have, and every wave is done with stage c
-    LQ_WAIT_VM(6);
-    __builtin_amdgcn_s_barrier();
   }
-  LQ_WAIT_VM(0);
+  LQ_WAIT_VM(0);  // no load to LDS is on its way when the sums go there
 
-  // lane holds weight rows wn*128 + 16i + 4t + v, token m0 + wm*64 + 16j + r
-  if constexpr (!SWIGLU) {
+  // The sums, four weight tiles at a time (SwiGLU: two gate tiles and the up tiles of the same columns): sum (ii, j) of a
+  // wave at (ii * 4 + j) KB of its 16 KB; unit q = wk, wk + WK, .. of 8 is two weight tiles of token tile q % 4.
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int m = m0 + wm * 64 + 16 * j + r;
-      if (m >= a.M) continue;
+  for (int half = 0; half < 2; ++half) {
+    __syncthreads();
+    uint8_t* mine = smem + wave * kRedWave + lane * 16;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int n = n0 + wn * 128 + 16 * i + 4 * t;
-        if (n >= a.N) continue;
-        f32x4 v = f32x4{acc[i][j][0] * a.alpha, acc[i][j][1] * a.alpha, acc[i][j][2] * a.alpha, acc[i][j][3] * a.alpha};
-        f32x4* dst = reinterpret_cast<f32x4*>(a.y + static_cast<size_t>(m) * a.ldy + n);
-        if (a.accumulate) {
-          const f32x4 o = *dst;
-          v = f32x4{o[0] + v[0], o[1] + v[1], o[2] + v[2], o[3] + v[3]};
-        }
-        *dst = v;
-      }
+    for (int ii = 0; ii < 4; ++ii) {
+      const int i = SWIGLU ? (ii & 1) * 4 + half * 2 + (ii >> 1) : half * 4 + ii;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) *reinterpret_cast<f32x4*>(mine + (ii * 4 + j) * 1024) = acc[i][j];
     }
-  } else {
-    // The up waves (wn = 1) hand alpha_up * acc to the gate waves (wn = 0) through LDS, four weight tiles at a
-    // time (64 KB): element (i, j, v) of lane L of token quarter wm at ((wm * 4 + ih) * 16 + j * 4 + v) * 64 + L.
-    float* xch = reinterpret_cast<float*>(smem);
+    __syncthreads();
 #pragma unroll
-    for (int half = 0; half < 2; ++half) {
-      __syncthreads();
-      if (wn == 1) {
+    for (int q0 = 0; q0 < 8; q0 += WK) {
+      const int q = q0 + wk, pair = q >> 2, j = q & 3;
+      f32x4 sum[2];
 #pragma unroll
-        for (int ih = 0; ih < 4; ++ih)
+      for (int h = 0; h < 2; ++h) {
+        const uint8_t* from = smem + wm * WK * kRedWave + ((2 * pair + h) * 4 + j) * 1024 + lane * 16;
+        sum[h] = *reinterpret_cast<const f32x4*>(from);
 #pragma unroll
-          for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int v = 0; v < 4; ++v)
-              xch[((wm * 4 + ih) * 16 + j * 4 + v) * 64 + lane] = acc[half * 4 + ih][j][v] * a.alpha2;
+        for (int k = 1; k < WK; ++k) sum[h] = sum[h] + *reinterpret_cast<const f32x4*>(from + k * kRedWave);
       }
-      __syncthreads();
-      if (wn == 0) {
+      const int m = m0 + 16 * j + r;
+      if constexpr (SWIGLU) {
 #pragma unroll
-        for (int ih = 0; ih < 4; ++ih) {
-          const int i = half * 4 + ih;
-          const int ncol = n0 + 16 * i;  // the block's first output column
+        for (int e = 0; e < 4; ++e) sum[1][e] *= a.alpha2;
+        put_swiglu(a, m, n0 + 16 * (half * 2 + pair), t, sum[0], sum[1]);
+      } else if (m < a.M) {
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            float v[4], amax = 0.f;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const float gv = acc[i][j][e] * a.alpha;
-              const float uv = xch[((wm * 4 + ih) * 16 + j * 4 + e) * 64 + lane];
-              v[e] = bf16_to_f32(f32_to_bf16((gv / (1.f + __expf(-gv))) * uv));
-              amax = fmaxf(amax, fabsf(v[e]));
-            }
-            // the block's 16 values are in lanes r, r + 16, r + 32, r + 48 (t = 0 .. 3)
-            amax = fmaxf(amax, __shfl_xor(amax, 16));
-            amax = fmaxf(amax, __shfl_xor(amax, 32));
-            const float sraw = a.gscale_out * (amax * (1.f / 6.f));
-            const uint32_t sc = __builtin_amdgcn_cvt_pk_fp8_f32(fminf(sraw, 448.f), 0.f, 0, false) & 0xffu;
-            const float sv = e4m3_to_f32(sc);
-            const float os = sv != 0.f ? 1.f / (sv * (1.f / a.gscale_out)) : 0.f;
-            const int m = m0 + wm * 64 + 16 * j + r;
-            if (m < a.M && ncol < a.N) {
-              uint8_t* qr = a.q_out + static_cast<size_t>(m) * (a.N / 2) + ncol / 2 + 2 * t;
-              const uint32_t b0 = e2m1x2_rne(v[0] * os, v[1] * os);
-              const uint32_t b1 = e2m1x2_rne(v[2] * os, v[3] * os);
-              *reinterpret_cast<uint16_t*>(qr) = static_cast<uint16_t>(b0 | (b1 << 8));
-              if (t == 0) a.sf_out[static_cast<size_t>(m) * (a.N / 16) + ncol / 16] = static_cast<uint8_t>(sc);
-            }
-          }
-        }
+        for (int h = 0; h < 2; ++h) put_out(a, m, n0 + 16 * (half * 4 + 2 * pair + h) + 4 * t, sum[h]);
       }
     }
   }
+}
+
+template <bool SWIGLU, int WM>
+int tile_launch(Nvfp4Args a, const char* name, hipStream_t s) {
+  a.tiles_m = cdiv(a.M, 64 * WM);
+  a.tiles_n = a.N / (SWIGLU ? 64 : 128);
+  constexpr int lds = 8 * kRedWave;
+  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_nvfp4_kernel<SWIGLU, WM>),
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  if (attr != hipSuccess) return fail(LQ_ERR_LAUNCH, std::string(name) + ": " + hipGetErrorString(attr));
+  hipLaunchKernelGGL((prefill_nvfp4_kernel<SWIGLU, WM>),
+                     dim3(static_cast<unsigned>(a.tiles_m) * static_cast<unsigned>(a.tiles_n)), dim3(kThreads), lds, s, a);
+  return check_launch(name);
+}
+
+// The tile height, by an estimate of the time: rounds of one tile per CU, each of which takes every wave of a K group
+// through its share of the chunks and then the sums. A higher tile reads its weights fewer times and its chunk costs a
+// little less, a lower one leaves fewer CUs idle and pads fewer tokens. Measured (us at WM = 1, 2, 4): 100 x 5120 x 5120
+// 21, 34, 60; 300 x 5120 x 17408 67, 111, 195; 500 x 17408 x 5120 114, 116, 133; 2048 x 5120 x 17408 321, 340, 412;
+// 4096 x 7168 x 5120 294, 264, 275; SwiGLU 2048 x 17408 x 5120 721, 650, 637 and 1000 x 3072 x 1024 27, 26, 21. The
+// estimate is within 10 % of these. (WM = 8, no K split: 262 at 4096 x 7168 x 5120, slower elsewhere.)
+int choose_wm(int M, int tiles_n, int C, long long cus) {
+  struct Kind {
+    int wm;
+    double chunk, tile;  // microseconds
+  };
+  int best_wm = 1;
+  double best = 0.;
+  for (const Kind& k : {Kind{1, 3.45, 5.}, Kind{2, 3.2, 5.}, Kind{4, 3.2, 6.}}) {
+    const long long rounds = (static_cast<long long>(tiles_n) * cdiv(M, 64 * k.wm) + cus - 1) / cus;
+    const double us = static_cast<double>(rounds) * (cdiv(C, 8 / k.wm) * k.chunk + k.tile);
+    if (k.wm == 1 || us < best) {
+      best = us;
+      best_wm = k.wm;
+    }
+  }
+  return best_wm;
 }
 
 template <bool SWIGLU>
@@ -286,16 +320,13 @@ int nvfp4_launch(Nvfp4Args a, const char* name, hipStream_t s) {
     return fail(LQ_ERR_ARG, nm + ": null pointer");
   if (!SWIGLU && reinterpret_cast<uintptr_t>(a.y) % 16 != 0) return fail(LQ_ERR_ARG, nm + ": y must be 16-byte aligned");
   a.C = a.K / 128;
-  a.rows_per_tile = SWIGLU ? 128 : kBN;
-  a.tiles_m = cdiv(a.M, kBM);
-  a.tiles_n = cdiv(a.N, a.rows_per_tile);
-  const long long blocks = static_cast<long long>(a.tiles_m) * a.tiles_n;
-  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_nvfp4_kernel<SWIGLU>),
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, kStages * kStage);
-  if (attr != hipSuccess) return fail(LQ_ERR_LAUNCH, nm + ": " + hipGetErrorString(attr));
-  hipLaunchKernelGGL((prefill_nvfp4_kernel<SWIGLU>), dim3(static_cast<unsigned>(blocks)), dim3(kThreads),
-                     kStages * kStage, s, a);
-  return check_launch(name);
+  int dev = 0;
+  (void)hipGetDevice(&dev);
+  switch (choose_wm(a.M, a.N / (SWIGLU ? 64 : 128), a.C, device_cus(dev))) {
+    case 1: return tile_launch<SWIGLU, 1>(a, name, s);
+    case 2: return tile_launch<SWIGLU, 2>(a, name, s);
+    default: return tile_launch<SWIGLU, 4>(a, name, s);
+  }
 }
 
 }  // namespace

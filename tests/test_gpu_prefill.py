@@ -361,6 +361,23 @@ def test_prefill_nvfp4(L, M, N, K):
     check_f32_tight(b[:, :N].astype(np.float64), ref + 0.5, "nvfp4 prefill accumulate")
 
 
+# one shape for each tile height (64, 128 and 256 tokens), last tiles of a few rows; fewer, as many and more chunks than
+# a K group has waves, with remainders
+@pytest.mark.parametrize("M,N", [(65, 128), (260, 8320), (1030, 6528)])
+@pytest.mark.parametrize("K", [128, 896, 1152])
+def test_prefill_nvfp4_tile_heights(L, M, N, K):
+    wv, ws, xq, xs = _nvfp4_operands(L, M, N, K, 140 + M)
+    raw = L.retile_nvfp4(to_dev(wv), to_dev(ws))
+    y = L.prefill_gemm_nvfp4(to_dev(xq), to_dev(xs), raw, 0.37, N).cpu().numpy()
+    rows = np.unique(np.r_[0, 15, 16, 63, 64, M // 2, M - 2, M - 1])
+    check_f32_tight(y[rows].astype(np.float64), O.prefill_nvfp4_rows(xq, xs, rows, wv, ws, 0.37), f"M={M} N={N} K={K}")
+    # gate = up = the same matrix: the FFN entry against this call's outputs and the quantizer
+    q, sf = L.prefill_swiglu_nvfp4(to_dev(xq), to_dev(xs), raw, 0.37, raw, 0.37, N, 0.05)
+    rq, rsf = L.silu_mul_quant_nvfp4(to_dev(y), to_dev(y), 0.05)
+    # (the same sums in another K split can move a value across a rounding boundary)
+    assert (q != rq).float().mean().item() <= 3e-3 and (sf != rsf).float().mean().item() <= 1e-3
+
+
 def test_prefill_nvfp4_device_quantized_activations(L):
     """The activations from quant_act_nvfp4 on the GPU, a larger shape, every 16th row checked."""
     M, N, K = 1024, 2048, 2048
