@@ -29,7 +29,7 @@
 //
 // What bounds it: the dequantization and the MFMAs share the SIMD's issue (3 VALU instructions per MFMA). Tiles of 256 x
 // 256 over 8 waves, which read a step's word from LDS just ahead of its use, took 430 us at 300 x 5120 x 17408 (40 tiles
-// on 256 CUs), 447 at 2048 x 5120 x 17408 and 760 for SwiGLU at 2048 x 17408 x 5120: now 67, 321 and 637.
+// on 256 CUs), 447 at 2048 x 5120 x 17408 and 760 for SwiGLU at 2048 x 17408 x 5120: now 60, 318 and 637.
 #include "lq_common.hpp"
 
 #include <string>
@@ -198,6 +198,10 @@ __global__ void __launch_bounds__(kThreads) prefill_nvfp4_kernel(const Nvfp4Args
   const int last = a.C - 1;
 #pragma unroll
   for (int v = 0; v < kLoads; ++v) issue_one(min(wk, last), v);
+  // A SIMD's two waves at different issue priority: one multiplies while the other takes in its next chunk, where equals
+  // drift into doing the same at once (300 x 5120 x 17408 62.1 -> 60.2 us, 300 x 17408 x 5120 SwiGLU 139 -> 134, 2048 x
+  // 17408 x 5120 level).
+  if (wave >= 4) __builtin_amdgcn_s_setprio(1);
   for (int c = wk; c < a.C; c += WK) {
     LQ_WAIT_VM(0);
     u32x4 aw[8], bw[4];
@@ -231,6 +235,7 @@ __global__ void __launch_bounds__(kThreads) prefill_nvfp4_kernel(const Nvfp4Args
     }
   }
   LQ_WAIT_VM(0);  // no load to LDS is on its way when the sums go there
+  __builtin_amdgcn_s_setprio(0);
 
   // The sums, four weight tiles at a time (SwiGLU: two gate tiles and the up tiles of the same columns): sum (ii, j) of a
   // wave at (ii * 4 + j) KB of its 16 KB; unit q = wk, wk + WK, .. of 8 is two weight tiles of token tile q % 4.
