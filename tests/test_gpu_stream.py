@@ -234,6 +234,36 @@ def test_to_half_rows_row_widths(L, K):
     assert np.array_equal(binv.cpu().numpy(), winv2)
 
 
+@pytest.mark.parametrize("K", [8, 520, 8192, 8200, 16392, 32768])
+def test_row_copies_in_pieces(L, K):
+    """Rows in 16-byte pieces (one, two and four a thread, ragged last waves) against the oracle, and the same values from
+    pointers that are not 16-byte aligned, which take the kernels of 2- and 4-byte loads."""
+    x = O.normal_f32(17 + K, 1.0, (3, K))
+    wh, winv = O.to_half_rows(x)
+    w = O.normal_bf16(18 + K, 0.1, (K,))
+    ro, _, _ = O.rmsnorm_half(x, w, 1e-6, True)
+    xb = O.f32_to_bf16(x)
+    wh2, _ = O.to_half_rows(O.bf16_to_f32(xb))
+    for off in (0, 1):
+        def at(t):
+            buf = torch.empty(t.numel() + 8, dtype=t.dtype, device=t.device)
+            v = buf[off:off + t.numel()].view(t.shape)
+            v.copy_(t)
+            return v
+        xd = at(to_dev(x))
+        xh, xinv = L.to_half_rows(xd)
+        assert np.array_equal(xh.view(torch.int16).cpu().numpy().view(np.uint16), wh)
+        assert np.array_equal(xinv.cpu().numpy(), winv)
+        bh, _ = L.bf16_to_half_rows(at(bf16_dev(xb)))
+        assert np.array_equal(bh.view(torch.int16).cpu().numpy().view(np.uint16), wh2)
+        out, nh, ninv = L.rmsnorm_half(xd, bf16_dev(w), 1e-6, True)
+        o = out.cpu().numpy()
+        assert np.max(np.abs(o - ro) / (np.abs(ro) + 1e-6 * np.abs(ro).max())) <= 1e-5
+        ch, ci = O.to_half_rows(o)  # the FP16 copy is exactly that of the device's own FP32 output
+        assert np.array_equal(nh.view(torch.int16).cpu().numpy().view(np.uint16), ch)
+        assert np.array_equal(ninv.cpu().numpy(), ci)
+
+
 def reference_style_weights(seed, N, K):
     """tests/stream_tests.cu:147-160: random bytes (no E4M3 NaN), NVFP4 scales 0x28..0x48, x with outliers."""
     rng = np.random.default_rng(seed)
