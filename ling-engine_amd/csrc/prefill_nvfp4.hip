@@ -12,7 +12,7 @@
 // accumulation across all of K; alpha is applied at the end.
 //
 //  * A wave computes 128 weight rows x 64 tokens (8 x 4 MFMA tiles, 128 accumulator registers; SwiGLU: 64 gate rows and
-//    the same 64 up rows). Per 128-value chunk a lane holds the raw 16 bytes (32 E2M1 values) and the 2 scales of its
+//    the same 64 up rows; NI = 4: 64 rows, for calls with few tiles). Per 128-value chunk a lane holds the raw 16 bytes (32 E2M1 values) and the 2 scales of its
 //    row for each of its 8 weight tiles and 4 token tiles, and dequantizes one 8-value step at a time: lane (r, t)
 //    supplies K 32t + 8s .. +8 at step s for both operands (a permutation of K inside the chunk, harmless as both
 //    operands use it; the weights' tiled layout holds exactly these 16 bytes per (row, t), slot r * 4 + t).
@@ -23,7 +23,7 @@
 //  * Nothing is shared while a wave computes, so there are no barriers: each wave streams its own operands to its own
 //    13.5 KB of LDS by direct loads, takes a landed chunk into registers (60 of them) and at once has the next one loaded
 //    over it, which then has the whole chunk's 128 MFMAs to arrive.
-//  * LDS of a wave: [weight values 128 x 64 B][weight scales 128 x 8][token values 64 x 64][token scales 64 x 8]. The
+//  * LDS of a wave (NI = 8): [weight values 128 x 64 B][weight scales 128 x 8][token values 64 x 64][token scales 64 x 8]. The
 //    16-byte units of a 64-byte row are XOR-swizzled by swz4(row) so the 16-byte fragment reads are conflict free whether
 //    the LDS serves 8 or 16 lanes of them per cycle; four lanes of a load read one run of 64 bytes.
 //
@@ -38,9 +38,9 @@ namespace lq {
 namespace {
 
 constexpr int kThreads = 512;
-constexpr int kWaveOffX = 128 * 72, kWaveStage = kWaveOffX + 64 * 72;  // a wave's LDS: weights, then tokens
+constexpr int wave_off_x(int ni) { return ni * 16 * 72; }  // a wave's LDS: 16 ni weight rows, then 64 tokens
 constexpr int kRedWave = 16 * 1024;  // a wave's sums of four weight tiles x four token tiles
-static_assert(kRedWave >= kWaveStage, "the reduction takes the larger part of LDS");
+static_assert(kRedWave >= wave_off_x(8) + 64 * 72, "the reduction takes the larger part of LDS");
 
 // 16 lanes read one 16-byte unit each of rows r .. r + 15 (r % 16 == 0): banks (row % 4, unit) must be distinct
 // over the 16 rows, and (row % 2, unit) over each aligned 8.
@@ -125,9 +125,11 @@ __device__ __forceinline__ void put_swiglu(const Nvfp4Args& a, int m, int ncol, 
   }
 }
 
-template <bool SWIGLU, int WM>
+template <bool SWIGLU, int NI, int WM>
 __global__ void __launch_bounds__(kThreads) prefill_nvfp4_kernel(const Nvfp4Args a) {
-  constexpr int WK = 8 / WM, TN = SWIGLU ? 64 : 128, TM = 64 * WM;
+  constexpr int WK = 8 / WM, TN = SWIGLU ? 64 : 16 * NI, TM = 64 * WM;
+  constexpr int kOffS = NI * 1024, kOffX = wave_off_x(NI);
+  static_assert(NI == 8 || (NI == 4 && !SWIGLU), "weight tiles of a wave");
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, t = lane >> 4;
@@ -152,7 +154,7 @@ __global__ void __launch_bounds__(kThreads) prefill_nvfp4_kernel(const Nvfp4Args
   const __amdgpu_buffer_rsrc_t sr2 = rsrc(SWIGLU ? (a.wsf2 ? a.wsf2 : a.w2) : (a.wsf ? a.wsf : a.w), sbytes);
   const __amdgpu_buffer_rsrc_t xr = rsrc(a.xq, a.M * (a.K / 2)), xsr = rsrc(a.xs, a.M * (a.K / 16));
 
-  // Weight rows are whole tiles of a matrix with N % 128 == 0: always in range. Weight tile i (0 .. 7) of the wave is
+  // Weight rows are whole tiles of a matrix with N % 128 == 0: always in range. Weight tile i of the wave is
   // 16-row tile n0 / 16 + i (SwiGLU: + i % 4, the up matrix from i = 4); a lane loads unit lane % 4 of row lane / 4 of a
   // tile's values, 4 bytes of two tiles' scales.
   const int srow = lane >> 2, su = (lane & 3) ^ swz4(srow);
@@ -171,27 +173,27 @@ __global__ void __launch_bounds__(kThreads) prefill_nvfp4_kernel(const Nvfp4Args
     const int m = m0 + 32 * j + (lane >> 1);
     xssrc[j] = m < a.M ? static_cast<unsigned>(m * (a.K / 16) + (lane & 1) * 4) : kOob;
   }
-  uint8_t* lds = smem + wave * kWaveStage;
-  // load v of a chunk's 18
-  constexpr int kLoads = 18;
+  uint8_t* lds = smem + wave * (kOffX + 64 * 72);
+  // load v of a chunk's
+  constexpr int kW = NI, kWS = kW + NI / 2, kX = kWS + 4, kLoads = kX + 2;
   auto issue_one = [&](int c, int v) {
-    if (v < 8) {
+    if (v < kW) {
       if (SWIGLU && v >= 4) dma16(wr2, lds + v * 1024, wsrc, wbase + (v - 4) * tstep + c * blkb);
       else dma16(wr1, lds + v * 1024, wsrc, wbase + v * tstep + c * blkb);
-    } else if (v < 12) {
-      const int p = v - 8;
-      if (SWIGLU && p >= 2) dma4(sr2, lds + 128 * 64 + p * 256, ssrc, sbase + 2 * (p - 2) * sstep + c * sblk);
-      else dma4(sr1, lds + 128 * 64 + p * 256, ssrc, sbase + 2 * p * sstep + c * sblk);
-    } else if (v < 16) {
-      dma16(xr, lds + kWaveOffX + (v - 12) * 1024, xsrc[v - 12], c * 64);
+    } else if (v < kWS) {
+      const int p = v - kW;
+      if (SWIGLU && p >= 2) dma4(sr2, lds + kOffS + p * 256, ssrc, sbase + 2 * (p - 2) * sstep + c * sblk);
+      else dma4(sr1, lds + kOffS + p * 256, ssrc, sbase + 2 * p * sstep + c * sblk);
+    } else if (v < kX) {
+      dma16(xr, lds + kOffX + (v - kWS) * 1024, xsrc[v - kWS], c * 64);
     } else {
-      dma4(xsr, lds + kWaveOffX + 64 * 64 + (v - 16) * 256, xssrc[v - 16], c * 8);
+      dma4(xsr, lds + kOffX + 64 * 64 + (v - kX) * 256, xssrc[v - kX], c * 8);
     }
   };
 
-  f32x4 acc[8][4];
+  f32x4 acc[NI][4];
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
+  for (int i = 0; i < NI; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
@@ -204,17 +206,17 @@ __global__ void __launch_bounds__(kThreads) prefill_nvfp4_kernel(const Nvfp4Args
   if (wave >= 4) __builtin_amdgcn_s_setprio(1);
   for (int c = wk; c < a.C; c += WK) {
     LQ_WAIT_VM(0);
-    u32x4 aw[8], bw[4];
-    f16x2 as[8], bs[4];
+    u32x4 aw[NI], bw[4];
+    f16x2 as[NI], bs[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      bw[j] = *reinterpret_cast<const u32x4*>(lds + kWaveOffX + val_off(16 * j + r, t));
-      bs[j] = scale_pair(*reinterpret_cast<const uint16_t*>(lds + kWaveOffX + 64 * 64 + (16 * j + r) * 8 + t * 2));
+      bw[j] = *reinterpret_cast<const u32x4*>(lds + kOffX + val_off(16 * j + r, t));
+      bs[j] = scale_pair(*reinterpret_cast<const uint16_t*>(lds + kOffX + 64 * 64 + (16 * j + r) * 8 + t * 2));
     }
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < NI; ++i) {
       aw[i] = *reinterpret_cast<const u32x4*>(lds + val_off(16 * i + r, t));
-      as[i] = scale_pair(*reinterpret_cast<const uint16_t*>(lds + 128 * 64 + (16 * i + r) * 8 + t * 2));
+      as[i] = scale_pair(*reinterpret_cast<const uint16_t*>(lds + kOffS + (16 * i + r) * 8 + t * 2));
     }
     // every read has returned before the next chunk's loads go over them (past the end the last chunk again, never read)
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -225,9 +227,9 @@ __global__ void __launch_bounds__(kThreads) prefill_nvfp4_kernel(const Nvfp4Args
 #pragma unroll
       for (int j = 0; j < 4; ++j) bf[j] = deq_word(bw[j][s], bs[j], s);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        // (one or two of the loads per weight tile: a burst would hold the wave up)
-        if (s * 8 + i < kLoads) issue_one(next, s * 8 + i);
+      for (int i = 0; i < NI; ++i) {
+        // (one of the loads per weight tile: a burst would hold the wave up)
+        if (s * NI + i < kLoads) issue_one(next, s * NI + i);
         const u32x4 af = deq_word(aw[i][s], as[i], s);
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc[i][j] = mfma16x16x32(af, bf[j], acc[i][j], true);
@@ -240,7 +242,7 @@ __global__ void __launch_bounds__(kThreads) prefill_nvfp4_kernel(const Nvfp4Args
   // The sums, four weight tiles at a time (SwiGLU: two gate tiles and the up tiles of the same columns): sum (ii, j) of a
   // wave at (ii * 4 + j) KB of its 16 KB; unit q = wk, wk + WK, .. of 8 is two weight tiles of token tile q % 4.
 #pragma unroll
-  for (int half = 0; half < 2; ++half) {
+  for (int half = 0; half < NI / 4; ++half) {
     __syncthreads();
     uint8_t* mine = smem + wave * kRedWave + lane * 16;
 #pragma unroll
@@ -274,41 +276,47 @@ __global__ void __launch_bounds__(kThreads) prefill_nvfp4_kernel(const Nvfp4Args
   }
 }
 
-template <bool SWIGLU, int WM>
+template <bool SWIGLU, int NI, int WM>
 int tile_launch(Nvfp4Args a, const char* name, hipStream_t s) {
   a.tiles_m = cdiv(a.M, 64 * WM);
-  a.tiles_n = a.N / (SWIGLU ? 64 : 128);
+  a.tiles_n = a.N / (SWIGLU ? 64 : 16 * NI);
   constexpr int lds = 8 * kRedWave;
-  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_nvfp4_kernel<SWIGLU, WM>),
+  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_nvfp4_kernel<SWIGLU, NI, WM>),
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   if (attr != hipSuccess) return fail(LQ_ERR_LAUNCH, std::string(name) + ": " + hipGetErrorString(attr));
-  hipLaunchKernelGGL((prefill_nvfp4_kernel<SWIGLU, WM>),
+  hipLaunchKernelGGL((prefill_nvfp4_kernel<SWIGLU, NI, WM>),
                      dim3(static_cast<unsigned>(a.tiles_m) * static_cast<unsigned>(a.tiles_n)), dim3(kThreads), lds, s, a);
   return check_launch(name);
 }
 
-// The tile height, by an estimate of the time: rounds of one tile per CU, each of which takes every wave of a K group
-// through its share of the chunks and then the sums. A higher tile reads its weights fewer times and its chunk costs a
-// little less, a lower one leaves fewer CUs idle and pads fewer tokens. Measured (us at WM = 1, 2, 4): 100 x 5120 x 5120
-// 21, 34, 60; 300 x 5120 x 17408 67, 111, 195; 500 x 17408 x 5120 114, 116, 133; 2048 x 5120 x 17408 321, 340, 412;
-// 4096 x 7168 x 5120 294, 264, 275; SwiGLU 2048 x 17408 x 5120 721, 650, 637 and 1000 x 3072 x 1024 27, 26, 21. The
-// estimate is within 10 % of these. (WM = 8, no K split: 262 at 4096 x 7168 x 5120, slower elsewhere.)
-int choose_wm(int M, int tiles_n, int C, long long cus) {
-  struct Kind {
-    int wm;
-    double chunk, tile;  // microseconds
-  };
-  int best_wm = 1;
-  double best = 0.;
-  for (const Kind& k : {Kind{1, 3.45, 5.}, Kind{2, 3.2, 5.}, Kind{4, 3.2, 6.}}) {
-    const long long rounds = (static_cast<long long>(tiles_n) * cdiv(M, 64 * k.wm) + cus - 1) / cus;
-    const double us = static_cast<double>(rounds) * (cdiv(C, 8 / k.wm) * k.chunk + k.tile);
-    if (k.wm == 1 || us < best) {
-      best = us;
-      best_wm = k.wm;
+// The tile, by an estimate of the time: rounds of one tile per CU, each of which takes every wave of a K group through its
+// share of the chunks and then the sums. A higher tile reads its weights fewer times and its chunk costs a little less, a
+// lower one leaves fewer CUs idle and pads fewer tokens; half the weight rows (NI = 4) dequantize more per MFMA, and pay
+// where whole wave tiles would leave half the CUs without work. Measured (us at WM = 1, 2, 4 with NI = 8, then NI = 4):
+// 100 x 5120 x 5120 21, 34, 60, 14; 200 x 2048 x 4096 18, 29, 50, 12; 160 x 5120 x 17408 56, 99, 186, 42; 200 x 5120 x
+// 5120 23, 35, 61, 26; 300 x 5120 x 17408 59, 100, 188, 74; 500 x 17408 x 5120 114, 116, 133; 2048 x 5120 x 17408 321, 340,
+// 412; 4096 x 7168 x 5120 294, 264, 275; SwiGLU 2048 x 17408 x 5120 721, 650, 637 and 1000 x 3072 x 1024 27, 26, 21. The
+// estimate is within 15 % of these. (WM = 8, no K split: 262 at 4096 x 7168 x 5120, slower elsewhere; NI = 4 with WM = 2
+// never ahead by more than 2 %.)
+struct TileKind {
+  int ni, wm;
+  double chunk, tile;  // microseconds
+};
+constexpr TileKind kKinds[] = {{8, 1, 3.45, 5.}, {8, 2, 3.2, 5.}, {8, 4, 3.2, 6.}, {4, 1, 2.15, 4.}};
+
+TileKind choose_tile(bool swiglu, int M, int N, int C, long long cus) {
+  TileKind best = kKinds[0];
+  double best_us = 0.;
+  for (const TileKind& k : kKinds) {
+    if (swiglu && k.ni != 8) continue;
+    const long long tiles = static_cast<long long>(N / (swiglu ? 64 : 16 * k.ni)) * cdiv(M, 64 * k.wm);
+    const double us = static_cast<double>((tiles + cus - 1) / cus) * (cdiv(C, 8 / k.wm) * k.chunk + k.tile);
+    if (&k == kKinds || us < best_us) {
+      best_us = us;
+      best = k;
     }
   }
-  return best_wm;
+  return best;
 }
 
 template <bool SWIGLU>
@@ -327,10 +335,13 @@ int nvfp4_launch(Nvfp4Args a, const char* name, hipStream_t s) {
   a.C = a.K / 128;
   int dev = 0;
   (void)hipGetDevice(&dev);
-  switch (choose_wm(a.M, a.N / (SWIGLU ? 64 : 128), a.C, device_cus(dev))) {
-    case 1: return tile_launch<SWIGLU, 1>(a, name, s);
-    case 2: return tile_launch<SWIGLU, 2>(a, name, s);
-    default: return tile_launch<SWIGLU, 4>(a, name, s);
+  const TileKind k = choose_tile(SWIGLU, a.M, a.N, a.C, device_cus(dev));
+  if constexpr (!SWIGLU)
+    if (k.ni == 4) return tile_launch<SWIGLU, 4, 1>(a, name, s);
+  switch (k.wm) {
+    case 1: return tile_launch<SWIGLU, 8, 1>(a, name, s);
+    case 2: return tile_launch<SWIGLU, 8, 2>(a, name, s);
+    default: return tile_launch<SWIGLU, 8, 4>(a, name, s);
   }
 }
 

@@ -361,11 +361,11 @@ def test_prefill_nvfp4(L, M, N, K):
     check_f32_tight(b[:, :N].astype(np.float64), ref + 0.5, "nvfp4 prefill accumulate")
 
 
-# one shape for each tile height (64, 128 and 256 tokens), last tiles of a few rows; fewer, as many and more chunks than
+# one shape for each tile (64 x 64, then 128 x 64, 128 x 128 and 128 x 256), last tiles of a few rows; fewer, as many and more chunks than
 # a K group has waves, with remainders
-@pytest.mark.parametrize("M,N", [(65, 128), (260, 8320), (1030, 6528)])
+@pytest.mark.parametrize("M,N", [(65, 128), (70, 8320), (260, 8320), (1030, 6528)])
 @pytest.mark.parametrize("K", [128, 896, 1152])
-def test_prefill_nvfp4_tile_heights(L, M, N, K):
+def test_prefill_nvfp4_tiles(L, M, N, K):
     wv, ws, xq, xs = _nvfp4_operands(L, M, N, K, 140 + M)
     raw = L.retile_nvfp4(to_dev(wv), to_dev(ws))
     y = L.prefill_gemm_nvfp4(to_dev(xq), to_dev(xs), raw, 0.37, N).cpu().numpy()
