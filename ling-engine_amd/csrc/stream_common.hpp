@@ -115,29 +115,37 @@ constexpr int kNT = 2;  // slc: streaming (non-temporal) weights
 
 template <int WF, int T>
 __device__ __forceinline__ void load_w(WRegs<WF, T>& R, const __amdgpu_buffer_rsrc_t (&rs)[T], const int (&toff)[T],
-                                       const int (&coff)[T], int c, int lane_off, int slot, unsigned oob) {
+                                       int c, int lane_off) {
 #pragma unroll
   for (int i = 0; i < T; ++i) {
     if constexpr (WF == kFp8) {
       const int so = toff[i] + c * kTileBytesFp8;
       R.v[i][0] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs[i], lane_off, so, kNT));
       R.v[i][1] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs[i], lane_off + 512, so, kNT));
-    } else if constexpr (WF == kFp4) {
-      const int so = toff[i] + c * kTileBytesFp4;
-      R.v[i][0] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs[i], lane_off, so, kNT));
-      R.sc[i] = static_cast<uint16_t>(
-          __builtin_amdgcn_raw_buffer_load_b16(rs[i], static_cast<int>((1024 + 2 * slot) | oob), so, 0));
     } else {
-      const int so = toff[i] + c * kValueBytesFp4;
+      const int so = toff[i] + c * (WF == kFp4 ? kTileBytesFp4 : kValueBytesFp4);
       R.v[i][0] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs[i], lane_off, so, kNT));
-      // slot s < 32: low byte at 2s, high nibble in the low half of byte 64 + s; slot 32 + L: byte 2L + 1
-      // and the high half of byte 64 + L (reference src/core/stream_gemm.cu:740-780).
-      const int L = slot & 31, hi = slot >> 5, cso = coff[i] + c * kCodeBytesFp4;
-      const uint32_t lo = __builtin_amdgcn_raw_buffer_load_b8(rs[i], static_cast<int>((2 * L + hi) | oob), cso, 0);
-      const uint32_t nb = __builtin_amdgcn_raw_buffer_load_b8(rs[i], static_cast<int>((64 + L) | oob), cso, 0);
-      R.sc[i] = lo | (((nb >> (4 * hi)) & 15u) << 8);
     }
   }
+}
+
+// NVFP4 scale bytes of a wave's four tiles and one chunk: one 8-byte load per lane (lane l has piece l % 16 of tile l / 16:
+// 16 pieces of raw scales, 12 of codes), which go through the wave's 512 bytes of LDS to the lanes that use them. They are
+// loaded and stored with the chunk's activations, a chunk ahead of their use. (Loaded by the lanes that use them they were
+// four 2-byte loads per chunk, coded eight of one byte, on the path that the weight stream shares: coded 17408 x 5120 at
+// M = 1 20.4 -> 18.5 us, 5120 x 25600 at M = 16 25.6 -> 22.5; raw 16.8 -> 16.5 and 20.4 -> 20.0 at M = 16.)
+__device__ __forceinline__ u32x2 load_scales(const __amdgpu_buffer_rsrc_t& rs, int soff, int lane_off, unsigned oob) {
+  return __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rs, static_cast<int>(lane_off | oob), soff, 0));
+}
+// Tile i's scale pair (raw) or 12-bit code pair for the lane of `slot`, from the wave's LDS bytes.
+template <int WF>
+__device__ __forceinline__ uint32_t read_scales(const uint8_t* sc, int i, int slot) {
+  const uint8_t* b = sc + i * 128;
+  if constexpr (WF == kFp4) return *reinterpret_cast<const uint16_t*>(b + 2 * slot);
+  // slot s < 32: low byte at 2s, high nibble in the low half of byte 64 + s; slot 32 + L: byte 2L + 1
+  // and the high half of byte 64 + L (reference src/core/stream_gemm.cu:740-780).
+  const int L = slot & 31, hi = slot >> 5;
+  return b[2 * L + hi] | (((b[64 + L] >> (4 * hi)) & 15u) << 8);
 }
 
 // The A operand of MFMA step s (8 weights, K 32t + 8s .. +8) for tile i.
@@ -357,7 +365,8 @@ template <int WF, int T, bool PAIR>
 struct SegTiles {
   int mi, wtile0;
   __amdgpu_buffer_rsrc_t rs[T];
-  int toff[T], coff[T];
+  int toff[T];
+  int soff, slane;  // NVFP4: the scale bytes of the wave's first tile, and the lane's piece of the wave's tiles from there
 };
 
 template <int WF, int T, bool PAIR, bool ONE = false>
@@ -379,7 +388,18 @@ __device__ __forceinline__ void seg_tiles(const StreamArgs& a, int tg, int wave,
     const int blk = WF == kFp8 ? kTileBytesFp8 : WF == kFp4 ? kTileBytesFp4 : kValueBytesFp4;
     s.rs[i] = make_rsrc(pick(a.w, m));
     s.toff[i] = tile * a.C * blk;
-    s.coff[i] = (Nm / 16) * a.C * kValueBytesFp4 + tile * a.C * kCodeBytesFp4;
+  }
+  if constexpr (WF != kFp8) {
+    static_assert(T == 4 && !PAIR, "a wave's scale bytes: 16 lanes for each of four tiles of one matrix");
+    const int lane = static_cast<int>(threadIdx.x) & 63, piece = lane & 15, last = pick(a.N, mi) / 16 - 1;
+    const int t0 = min(s.wtile0, last), ahead = min(s.wtile0 + (lane >> 4), last) - t0;
+    if constexpr (WF == kFp4) {
+      s.soff = t0 * a.C * kTileBytesFp4 + kValueBytesFp4;
+      s.slane = ahead * a.C * kTileBytesFp4 + piece * 8;
+    } else {
+      s.soff = (last + 1) * a.C * kValueBytesFp4 + t0 * a.C * kCodeBytesFp4;
+      s.slane = piece < kCodeBytesFp4 / 8 ? ahead * a.C * kCodeBytesFp4 + piece * 8 : static_cast<int>(0x80000000u);
+    }
   }
 }
 
@@ -679,6 +699,7 @@ struct Smem {
   static constexpr int XS_BYTES = 16 * G * 256;  // one chunk of activations, 16G rows
   uint8_t xs[NSLOT][XS_BYTES];
   float xsc[NSLOT][16 * G];  // kCvt: 2^(e - 15) of each row's chunk in the slot
+  uint8_t sc[NSLOT][4][512];  // NVFP4: a chunk's scale bytes, each wave its own
   uint8_t tabs[kMaxMats][64];
   int last_flag[2];
 };

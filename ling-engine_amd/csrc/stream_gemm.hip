@@ -143,10 +143,13 @@ __device__ __forceinline__ void stream_body(const StreamArgs& a, int p, Smem<G>&
 
   WRegs<WF, T> wr[PF];
   u32x4 xr[PF][G];
+  u32x2 scr[PF];  // NVFP4: the lane's piece of the stage's scale bytes
   // Every ring load is issued unconditionally (the wait counts then hold on every path); a load past the
   // stream's end is turned into an out-of-range buffer load (offset >= num_records), which returns zeros and
   // touches no memory.
   auto load_x = [&](int j, int lcj, unsigned oob) {
+    if constexpr (WF != kFp8)
+      scr[j] = load_scales(L.rs[0], L.soff + lcj * (WF == kFp4 ? kTileBytesFp4 : kCodeBytesFp4), L.slane, oob);
 #pragma unroll
     for (int i = 0; i < G; ++i)
       xr[j][i] = __builtin_bit_cast(
@@ -169,7 +172,7 @@ __device__ __forceinline__ void stream_body(const StreamArgs& a, int p, Smem<G>&
     __builtin_amdgcn_sched_barrier(0);
     load_x(j, lc, oob);
     __builtin_amdgcn_sched_barrier(0);
-    load_w<WF, T>(wr[j], L.rs, L.toff, L.coff, lc, static_cast<int>(lane_off | oob), slot, oob);
+    load_w<WF, T>(wr[j], L.rs, L.toff, lc, static_cast<int>(lane_off | oob));
     __builtin_amdgcn_sched_barrier(0);
     advance();
   };
@@ -186,11 +189,12 @@ __device__ __forceinline__ void stream_body(const StreamArgs& a, int p, Smem<G>&
   };
   auto load_stage_w = [&](int j) {
     __builtin_amdgcn_sched_barrier(0);
-    load_w<WF, T>(wr[j], L.rs, L.toff, L.coff, lc, static_cast<int>(lane_off | stage_oob), slot, stage_oob);
+    load_w<WF, T>(wr[j], L.rs, L.toff, lc, static_cast<int>(lane_off | stage_oob));
     __builtin_amdgcn_sched_barrier(0);
     advance();
   };
   auto put_x = [&](int j, int sl) {
+    if constexpr (WF != kFp8) *reinterpret_cast<u32x2*>(sm.sc[sl][wave] + lane * 8) = scr[j];
 #pragma unroll
     for (int i = 0; i < G; ++i) {
       if constexpr (CVT) {
@@ -200,6 +204,16 @@ __device__ __forceinline__ void stream_body(const StreamArgs& a, int p, Smem<G>&
         *reinterpret_cast<u32x4*>(xs[sl] + xdst[i]) = xr[j][i];
       }
     }
+  };
+  auto scales = [&](uint32_t (&sc)[T], int sl) {
+    if constexpr (WF != kFp8)
+#pragma unroll
+      for (int i = 0; i < T; ++i) sc[i] = read_scales<WF>(sm.sc[sl][wave], i, slot);
+  };
+  auto take_scales = [&](WRegs<WF, T>& R, const uint32_t (&sc)[T]) {
+    if constexpr (WF != kFp8)
+#pragma unroll
+      for (int i = 0; i < T; ++i) R.sc[i] = sc[i];
   };
   // kCvt: a chunk's MFMA sums (accc) join the running sums (acc2) times the row's chunk scale.
   f32x4 accc[T][G];
@@ -294,7 +308,7 @@ __device__ __forceinline__ void stream_body(const StreamArgs& a, int p, Smem<G>&
       poob[c] = lleft > 0 ? 0u : 0x80000000u;
       plc[c] = lc;
       Lp[c] = L;
-      if (wave != 0) load_w<WF, T>(pr[c], L.rs, L.toff, L.coff, lc, static_cast<int>(lane_off | poob[c]), slot, poob[c]);
+      if (wave != 0) load_w<WF, T>(pr[c], L.rs, L.toff, lc, static_cast<int>(lane_off | poob[c]));
       advance();
     }
     int lcs[PF - 1];
@@ -305,7 +319,7 @@ __device__ __forceinline__ void stream_body(const StreamArgs& a, int p, Smem<G>&
       oobs[j] = lleft > 0 ? 0u : 0x80000000u;
       lcs[j] = lc;
       Lr[j] = L;
-      if (wave != 0) load_w<WF, T>(wr[j], L.rs, L.toff, L.coff, lc, static_cast<int>(lane_off | oobs[j]), slot, oobs[j]);
+      if (wave != 0) load_w<WF, T>(wr[j], L.rs, L.toff, lc, static_cast<int>(lane_off | oobs[j]));
       advance();
     }
     ready();
@@ -313,8 +327,7 @@ __device__ __forceinline__ void stream_body(const StreamArgs& a, int p, Smem<G>&
     if (wave == 0) {
 #pragma unroll
       for (int c = 0; c < NPRE; ++c)
-        load_w<WF, T>(pr[c], Lp[c].rs, Lp[c].toff, Lp[c].coff, plc[c], static_cast<int>(lane_off | poob[c]), slot,
-                      poob[c]);
+        load_w<WF, T>(pr[c], Lp[c].rs, Lp[c].toff, plc[c], static_cast<int>(lane_off | poob[c]));
     }
     // chunk c's image: 16G rows x 16 units of 16 bytes, as put_x lays it out (unit u of row m at u ^ (m & 15));
     // load k of wave w fills 64 consecutive units (rows 4 (4k + w) .. +4), each lane fetching the source unit that
@@ -332,8 +345,7 @@ __device__ __forceinline__ void stream_body(const StreamArgs& a, int p, Smem<G>&
     if (wave == 0) {
 #pragma unroll
       for (int j = 0; j < PF - 1; ++j)
-        load_w<WF, T>(wr[j], Lr[j].rs, Lr[j].toff, Lr[j].coff, lcs[j], static_cast<int>(lane_off | oobs[j]), slot,
-                      oobs[j]);
+        load_w<WF, T>(wr[j], Lr[j].rs, Lr[j].toff, lcs[j], static_cast<int>(lane_off | oobs[j]));
     }
 #pragma unroll
     for (int j = 0; j < PF - 1; ++j) load_x(j, lcs[j], oobs[j]);
@@ -363,7 +375,7 @@ __device__ __forceinline__ void stream_body(const StreamArgs& a, int p, Smem<G>&
     for (int j = 0; j < PF - 1; ++j) {
       oobs[j] = lleft > 0 ? 0u : 0x80000000u;
       lcs[j] = lc;
-      load_w<WF, T>(wr[j], L.rs, L.toff, L.coff, lc, static_cast<int>(lane_off | oobs[j]), slot, oobs[j]);
+      load_w<WF, T>(wr[j], L.rs, L.toff, lc, static_cast<int>(lane_off | oobs[j]));
       advance();
     }
     ready();
@@ -386,6 +398,8 @@ __device__ __forceinline__ void stream_body(const StreamArgs& a, int p, Smem<G>&
 #pragma unroll
     for (int s = 0; s < 4; ++s) read_b<G>(bc[s], xs[0], s, r, t);
     if constexpr (CVT) chunk_scales(scc, 0);
+    uint32_t wsc[T], wsn[T];
+    scales(wsc, 0);
     for (int base = 0; base < npad; base += PF) {
 #pragma unroll
       for (int j = 0; j < PF; ++j) {
@@ -398,7 +412,9 @@ __device__ __forceinline__ void stream_body(const StreamArgs& a, int p, Smem<G>&
 #pragma unroll
         for (int s = 0; s < 4; ++s) read_b<G>(bn[s], xs[sl], s, r, t);
         if constexpr (CVT) chunk_scales(scn, sl);
+        scales(wsn, sl);
         if (it < n_ring) {
+          take_scales(wr[j], wsc);
           const uint8_t* tab[T];
           tables(tab);
           if constexpr (CVT) {
@@ -421,6 +437,10 @@ __device__ __forceinline__ void stream_body(const StreamArgs& a, int p, Smem<G>&
 #pragma unroll
           for (int g = 0; g < G; ++g) scc[g] = scn[g];
         }
+        if constexpr (WF != kFp8) {
+#pragma unroll
+          for (int i = 0; i < T; ++i) wsc[i] = wsn[i];
+        }
       }
     }
   } else {
@@ -433,6 +453,9 @@ __device__ __forceinline__ void stream_body(const StreamArgs& a, int p, Smem<G>&
         __syncthreads();
         load_stage_w((j + PF - 1) % PF);
         if (it < n_ring) {
+          uint32_t wsc[T];
+          scales(wsc, it & 1);
+          take_scales(wr[j], wsc);
           const uint8_t* tab[T];
           tables(tab);
           if constexpr (CVT) {

@@ -356,6 +356,31 @@ def test_l2_prefetch_weights_changes_nothing(L):
         L.l2_prefetch_weights(tw, False, False, N, 100, 1 << 20)
 
 
+@pytest.mark.parametrize("M", [3, 20, 37])
+@pytest.mark.parametrize("N,K", [(16, 128), (272, 640), (1040, 384)])
+def test_stream_nvfp4_scale_bytes_of_ragged_tile_groups(L, N, K, M):
+    """A wave loads the scale bytes of its four tiles at once: matrices whose last tile group holds one tile of the 16, with
+    scales that differ from row to row and block to block, raw and coded, alone and beside another matrix."""
+    w = O.normal_bf16(90 + N, 0.02, (N, K))
+    v, s, g, _ = O.quant_nvfp4(w)
+    ok, table, code_of = O.scale_code_table(s)
+    assert ok
+    raw = L.retile_nvfp4(to_dev(v), to_dev(s))
+    blob, _ = L.retile_nvfp4_coded(to_dev(v), to_dev(s), to_dev(code_of))
+    xh, xinv = L.to_half_rows(to_dev(O.normal_f32(91, 1.0, (M, K))))
+    a = L.stream_gemm_nvfp4(xh, xinv, raw, None, g, N, K)
+    b = L.stream_gemm_nvfp4(xh, xinv, blob, to_dev(table), g, N, K)
+    xd = xh.view(torch.float16).cpu().numpy().astype(np.float64) * xinv.cpu().numpy()[:, None].astype(np.float64)
+    ref = xd @ O.dequant_nvfp4(v, s, g).astype(np.float64).T
+    rms = np.sqrt(np.mean(ref ** 2, axis=1, keepdims=True))
+    # exact products, FP32 sums of K <= 640 terms
+    assert np.max(np.abs(a.cpu().numpy() - ref) / rms) <= 1e-5
+    assert torch.equal(a, b)
+    y = [torch.empty((M, N), dtype=torch.float32, device=DEV) for _ in range(2)]
+    L.stream_gemm_multi(True, xh, xinv, [(blob, to_dev(table), g, y[0], N), (raw, None, g, y[1], N)], K)
+    assert torch.equal(y[0], a) and torch.equal(y[1], a)
+
+
 @pytest.mark.parametrize("N,K", [(4096, 2560), (8192, 5120)])
 def test_stream_gemm_gather_nvfp4_bit_exact(L, N, K):
     """The sparse head (reference tests/stream_tests.cu:271-300): a row subset, not in order, from the raw blob
