@@ -24,6 +24,7 @@
 //    token tile per group), so the workgroups running at once on an XCD share the K slices of both operands
 //    in its L2 instead of re-streaming the whole activation matrix per weight tile.
 #include "lq_common.hpp"
+#include "lq_prefill_offsets.hpp"
 #include "lq_workspace.hpp"
 
 #include <algorithm>
@@ -396,19 +397,16 @@ __global__ void __launch_bounds__(64 * WN * WM) prefill_tile_kernel(const Prefil
 
   // Load-to-LDS plan as in prefill_fp8_kernel: load i of wave w fills 8 rows from (i * NW + w) * 8. A row past the
   // operand gets an offset that is out of range by itself.
-  constexpr unsigned kOob = 0x80000000u;
-  unsigned wsrc[LW], xsrc[LX], ssrc = kOob;
+  unsigned wsrc[LW], xsrc[LX], ssrc = kLoadNothing;
 #pragma unroll
   for (int i = 0; i < LW; ++i) {
     const int row = (i * NW + wave) * 8 + (lane >> 3), u = (lane & 7) ^ swz(row), n = n0 + row;
-    wsrc[i] = n < a.N ? static_cast<unsigned>((n >> 4) * a.KB * kTileBytesFp8 +
-                                              (((((row & 15) >> 3) * 2 + (u >> 2)) * 8 + (row & 7)) * 4 + (u & 3)) * 16)
-                      : kOob;
+    wsrc[i] = n < a.N ? weight_unit_offset(n, u, a.KB) : kLoadNothing;
   }
 #pragma unroll
   for (int i = 0; i < LX; ++i) {
     const int row = (i * NW + wave) * 8 + (lane >> 3), u = (lane & 7) ^ swz(row), m = m0 + row;
-    xsrc[i] = m < a.M ? static_cast<unsigned>(m * a.K + u * 16) : kOob;
+    xsrc[i] = m < a.M ? activation_unit_offset(m, u, a.K) : kLoadNothing;
   }
   if constexpr (BLOCK) {
     const int row = wave * 64 + lane;
@@ -417,14 +415,15 @@ __global__ void __launch_bounds__(64 * WN * WM) prefill_tile_kernel(const Prefil
   // Loads [v0, v1) of a stage's kVm. (A block past the end is issued out of range: every wait count then holds on
   // every path.)
   auto issue_some = [&](int st, int kb, int v0, int v1) {
-    const unsigned oob = kb < a.KB ? 0u : kOob;
+    const unsigned oob = kb < a.KB ? 0u : kLoadNothing;
     uint8_t* base = smem + st * STG;
 #pragma unroll
     for (int v = v0; v < v1; ++v) {
-      if (v < LW) dma16(wr, base + (v * NW + wave) * 1024, wsrc[v] | oob, kb * kTileBytesFp8);
+      if (v < LW) dma16(wr, base + (v * NW + wave) * 1024, wsrc[v] | oob, block_offset(kb, a.KB, kTileBytesFp8));
       else if (v < LW + LX)
-        dma16(xr, base + TN * kRowBytes + ((v - LW) * NW + wave) * 1024, xsrc[v - LW] | oob, kb * kRowBytes);
-      else dma4(sr, base + (TN + TM) * kRowBytes + wave * 256, ssrc | oob, kb * 4);
+        dma16(xr, base + TN * kRowBytes + ((v - LW) * NW + wave) * 1024, xsrc[v - LW] | oob,
+              block_offset(kb, a.KB, kRowBytes));
+      else dma4(sr, base + (TN + TM) * kRowBytes + wave * 256, ssrc | oob, block_offset(kb, a.KB, 4));
     }
   };
   // all loads but those of the newest KEEP stages have landed

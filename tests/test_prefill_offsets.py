@@ -1,0 +1,74 @@
+"""Load offsets of the FP8 prefill kernels (ling-engine_amd/csrc/lq_prefill_offsets.hpp), compiled here for the host.
+A raw buffer load is out of range where vector offset >= bytes - scalar offset; for every lane, load and K block that a
+kernel issues, those past the operand's rows and blocks among them, the scalar offset has to stay within the operand (the
+difference never goes below zero), a load inside has to read its own 16 bytes, and a load outside has to be out of range."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+CSRC = os.path.join(os.path.dirname(HERE), "ling-engine_amd", "csrc")
+
+DRIVER = r"""
+#include <cstdio>
+#include "lq_prefill_offsets.hpp"
+using namespace lq;
+static long long tests = 0, bad = 0;
+static void expect(bool inside, unsigned v, unsigned s, unsigned width, unsigned bytes, unsigned want, const char* what,
+                   int a, int b) {
+  ++tests;
+  const bool ok = s <= bytes && (inside ? static_cast<unsigned long long>(v) + s == want && want + width <= bytes
+                                        : v >= bytes - s);
+  if (!ok && bad++ < 5) std::printf("%s: rows %d, row %d: v %u s %u of %u\n", what, a, b, v, s, bytes);
+}
+// where unit u of row n, block kb, lies: 16-row tiles of KB blocks of 2048 bytes, rows 8h + g, K pieces 32t + 16q
+static unsigned weight_at(int n, int u, int kb, int KB) {
+  const int h = (n % 16) / 8, g = n % 8, q = u / 4, t = u % 4;
+  return ((n / 16) * KB + kb) * 2048u + (((h * 2 + q) * 8 + g) * 4 + t) * 16u;
+}
+
+// the smaller tiles: loads of TN weight rows, TM tokens and their scales, blocks 0 .. KB - 1 + stages
+static void tile(int TN, int TM, int stages, int M, int N, int KB) {
+  const int K = KB * 128;
+  const unsigned wb = static_cast<unsigned>(N) * K, xb = static_cast<unsigned>(M) * K, sb = static_cast<unsigned>(M) * KB * 4;
+  for (int kb = 0; kb < KB + stages; ++kb) {
+    const unsigned past = kb < KB ? 0u : kLoadNothing;
+    for (int n0 = 0; n0 < N; n0 += TN)
+      for (int n = n0; n < n0 + TN; ++n)
+        for (int u = 0; u < 8; ++u)
+          expect(n < N && kb < KB, (n < N ? weight_unit_offset(n, u, KB) : kLoadNothing) | past, block_offset(kb, KB, 2048), 16,
+                 wb, weight_at(n, u, kb, KB), "tile weights", N, n);
+    for (int m0 = 0; m0 < M; m0 += TM)
+      for (int m = m0; m < m0 + TM; ++m) {
+        for (int u = 0; u < 8; ++u)
+          expect(m < M && kb < KB, (m < M ? activation_unit_offset(m, u, K) : kLoadNothing) | past, block_offset(kb, KB, 128),
+                 16, xb, static_cast<unsigned>(m * K + kb * 128 + u * 16), "tile activations", M, m);
+        expect(m < M && kb < KB, (m < M ? static_cast<unsigned>(m * KB * 4) : kLoadNothing) | past, block_offset(kb, KB, 4), 4,
+               sb, static_cast<unsigned>((m * KB + kb) * 4), "tile scales", M, m);
+      }
+  }
+}
+
+int main() {
+  const int ms[] = {1, 2, 3, 5, 63, 64, 65, 129, 200}, ns[] = {128, 256, 384}, kbs[] = {1, 2, 3, 5, 9};
+  const int shapes[][3] = {{64, 64, 4}, {128, 64, 3}, {128, 128, 4}, {128, 128, 2}};
+  for (int M : ms)
+    for (int N : ns)
+      for (int KB : kbs)
+        for (auto& s : shapes) tile(s[0], s[1], s[2], M, N, KB);
+  std::printf("tests %lld bad %lld\n", tests, bad);
+  return bad != 0 || tests < 100000;
+}
+"""
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
+def test_scalar_offsets_stay_within_the_operand(tmp_path):
+    src = tmp_path / "offsets.cpp"
+    exe = tmp_path / "offsets"
+    src.write_text(DRIVER)
+    subprocess.run(["g++", "-O2", "-std=c++17", "-Wall", "-I", CSRC, str(src), "-o", str(exe)], check=True)
+    out = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
+    assert out.returncode == 0, out.stdout + out.stderr
