@@ -164,14 +164,16 @@ __global__ void __launch_bounds__(kThreads) prefill_fp8_kernel(const PrefillArgs
 
   // Load-to-LDS plan: load i (0..3) of wave w writes LDS bytes [((i * 8 + w) * 64 + lane) * 16, +16) of an
   // operand tile: row = (i * 8 + w) * 8 + lane / 8, swizzled unit lane % 8, i.e. source unit u = lane % 8 ^ swz(row)
-  // (the same for every i, as i moves the row by 64). Weights: the row's 16-row tile tw and row rr in it; unit
-  // u = 4 q + tt is the tiled piece ((h*2 + q)*8 + g)*4 + tt (g = rr % 8, h = rr / 8); load i is 4 tiles on.
-  // Activations: row-major, load i is 64 rows on (a multiple of 16 rows: swz is the same). The per-i and per-block steps go in the scalar offset.
+  // (the same for every i, as i moves the row by 64, a multiple of 16). The per-i and per-block steps go in the scalar
+  // offset.
   const int row0 = wave * 8 + (lane >> 3), u0 = (lane & 7) ^ swz(row0);
-  const int wsrc = (((n0 >> 4) + (row0 >> 4)) * a.KB) * kTileBytesFp8 +
-                   (((((row0 & 15) >> 3) * 2 + (u0 >> 2)) * 8 + (row0 & 7)) * 4 + (u0 & 3)) * 16;
-  const int xsrc = (m0 + row0) * a.K + u0 * 16;
-  const int wstep = 4 * a.KB * kTileBytesFp8, xstep = 64 * a.K;
+  const unsigned wsrc = weight_unit_offset(n0 + row0, u0, a.KB), xsrc = activation_unit_offset(m0 + row0, u0, a.K);
+  unsigned wload[4], xload[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    wload[i] = load_offset(n0 + wave * 8, i, a.N, 64u * static_cast<unsigned>(a.K));
+    xload[i] = load_offset(m0 + wave * 8, i, a.M, 64u * static_cast<unsigned>(a.K));
+  }
   // activation scales: waves 0-3 load one token's scale per lane
   const int srow = wave * 64 + lane;
   const int ssrc = (wave < 4 && m0 + srow < a.M) ? (m0 + srow) * a.KB * 4 : static_cast<int>(0x80000000u);
@@ -183,11 +185,11 @@ __global__ void __launch_bounds__(kThreads) prefill_fp8_kernel(const PrefillArgs
     if (part < 2) {
 #pragma unroll
       for (int i = 2 * part; i < 2 * part + 2; ++i)
-        dma16(wr, base + (i * 8 + wave) * 1024, wsrc, kb * kTileBytesFp8 + i * wstep);
+        dma16(wr, base + (i * 8 + wave) * 1024, wsrc, kb * kTileBytesFp8 + wload[i]);
     } else if (part < 4) {
 #pragma unroll
       for (int i = 2 * (part - 2); i < 2 * (part - 2) + 2; ++i)
-        dma16(xr, base + kOpBytes + (i * 8 + wave) * 1024, xsrc, kb * kRowBytes + i * xstep);
+        dma16(xr, base + kOpBytes + (i * 8 + wave) * 1024, xsrc, kb * kRowBytes + xload[i]);
     } else if (BLOCK && wave < 4) {
       dma4(sr, base + 2 * kOpBytes + wave * 256, ssrc, kb * 4);
     }

@@ -1,7 +1,8 @@
 """Load offsets of the FP8 prefill kernels (ling-engine_amd/csrc/lq_prefill_offsets.hpp), compiled here for the host.
 A raw buffer load is out of range where vector offset >= bytes - scalar offset; for every lane, load and K block that a
 kernel issues, those past the operand's rows and blocks among them, the scalar offset has to stay within the operand (the
-difference never goes below zero), a load inside has to read its own 16 bytes, and a load outside has to be out of range."""
+difference never goes below zero), a load inside has to read its own bytes, and a load outside has to be out of range (the
+256 x 256 tile's may read other rows that exist)."""
 import os
 import shutil
 import subprocess
@@ -17,10 +18,11 @@ DRIVER = r"""
 using namespace lq;
 static long long tests = 0, bad = 0;
 static void expect(bool inside, unsigned v, unsigned s, unsigned width, unsigned bytes, unsigned want, const char* what,
-                   int a, int b) {
+                   int a, int b, bool any = false) {
   ++tests;
-  const bool ok = s <= bytes && (inside ? static_cast<unsigned long long>(v) + s == want && want + width <= bytes
-                                        : v >= bytes - s);
+  const unsigned long long at = static_cast<unsigned long long>(v) + s;
+  const bool ok = s <= bytes && (inside ? at == want && want + width <= bytes
+                                        : v >= bytes - s || (any && at + width <= bytes));
   if (!ok && bad++ < 5) std::printf("%s: rows %d, row %d: v %u s %u of %u\n", what, a, b, v, s, bytes);
 }
 // where unit u of row n, block kb, lies: 16-row tiles of KB blocks of 2048 bytes, rows 8h + g, K pieces 32t + 16q
@@ -51,6 +53,28 @@ static void tile(int TN, int TM, int stages, int M, int N, int KB) {
   }
 }
 
+// the 256 x 256 tile: waves of 8 rows, loads i = 0 .. 3 64 rows apart, over the rows that are there or not
+static void whole(int M, int N, int KB) {
+  const int K = KB * 128;
+  const unsigned wb = static_cast<unsigned>(N) * K, xb = static_cast<unsigned>(M) * K;
+  for (int kb = 0; kb < KB; ++kb)
+    for (int i = 0; i < 4; ++i)
+      for (int row = 0; row < 64; ++row)
+        for (int u = 0; u < 8; ++u) {
+          for (int n0 = 0; n0 < N; n0 += 256) {
+            const int n = n0 + row + 64 * i;
+            const unsigned s = kb * 2048u + load_offset(n0 + row / 8 * 8, i, N, 64u * K);
+            expect(n < N, weight_unit_offset(n0 + row, u, KB), s, 16, wb, weight_at(n, u, kb, KB), "weights", N, n, true);
+          }
+          for (int m0 = 0; m0 < M; m0 += 256) {
+            const int m = m0 + row + 64 * i;
+            const unsigned s = kb * 128u + load_offset(m0 + row / 8 * 8, i, M, 64u * K);
+            expect(m < M, activation_unit_offset(m0 + row, u, K), s, 16, xb, static_cast<unsigned>(m * K + kb * 128 + u * 16),
+                   "activations", M, m, true);
+          }
+        }
+}
+
 int main() {
   const int ms[] = {1, 2, 3, 5, 63, 64, 65, 129, 200}, ns[] = {128, 256, 384}, kbs[] = {1, 2, 3, 5, 9};
   const int shapes[][3] = {{64, 64, 4}, {128, 64, 3}, {128, 128, 4}, {128, 128, 2}};
@@ -58,6 +82,9 @@ int main() {
     for (int N : ns)
       for (int KB : kbs)
         for (auto& s : shapes) tile(s[0], s[1], s[2], M, N, KB);
+  for (int M : ms)
+    for (int N : ns)
+      for (int KB : kbs) whole(M, N, KB);
   std::printf("tests %lld bad %lld\n", tests, bad);
   return bad != 0 || tests < 100000;
 }
