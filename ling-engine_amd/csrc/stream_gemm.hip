@@ -369,6 +369,7 @@ __device__ __forceinline__ void stream_body(const StreamArgs& a, int p, Smem<G>&
     }
   } else if constexpr (XCOH) {
     // weights of the first stages first, then the wait for the activations, then their loads
+    static_assert(WF == kFp8, "load_x takes NVFP4 scales from the cursor L, which has moved on here");
     int lcs[PF - 1];
     unsigned oobs[PF - 1];
 #pragma unroll
