@@ -699,10 +699,15 @@ struct Smem {
   static constexpr int XS_BYTES = 16 * G * 256;  // one chunk of activations, 16G rows
   uint8_t xs[NSLOT][XS_BYTES];
   float xsc[NSLOT][16 * G];  // kCvt: 2^(e - 15) of each row's chunk in the slot
-  uint8_t sc[NSLOT][4][512];  // NVFP4: a chunk's scale bytes, each wave its own
   uint8_t tabs[kMaxMats][64];
   int last_flag[2];
 };
+template <int G>
+struct SmemFp4 : Smem<G> {
+  alignas(16) uint8_t sc[Smem<G>::NSLOT][4][512];  // a chunk's scale bytes, each wave its own
+};
+template <int G, int WF>
+using StreamSmem = std::conditional_t<WF == kFp8, Smem<G>, SmemFp4<G>>;
 
 // Body modes: kYCoh = the pair epilogue's stores write through (a later phase of the same launch reads them);
 // kXCoh = activations are read agent-coherently and only after `ready()` returns (the weight ring's first

@@ -64,7 +64,7 @@ namespace {
 // wave 0's weights in xpre.
 template <int G, int WF, int TW, bool F16, bool PAIR, bool OUTF32, int MODE, bool ONE = false, int NPRE = 0,
           class Ready>
-__device__ __forceinline__ void stream_body(const StreamArgs& a, int p, Smem<G>& sm, Ready&& ready,
+__device__ __forceinline__ void stream_body(const StreamArgs& a, int p, StreamSmem<G, WF>& sm, Ready&& ready,
                                             uint8_t* xpre = nullptr) {
   constexpr int T = TW;
   constexpr int PF = pf_stages<T>(G);
@@ -566,7 +566,7 @@ __device__ __forceinline__ void stream_body(const StreamArgs& a, int p, Smem<G>&
 
 template <int G, int WF, int TW, bool F16, bool PAIR, bool OUTF32, bool CVT = false, bool ONE = false>
 __global__ void __launch_bounds__(kThreads) stream_kernel(const StreamArgs a) {
-  __shared__ __attribute__((aligned(16))) Smem<G> sm;
+  __shared__ __attribute__((aligned(16))) StreamSmem<G, WF> sm;
   if (static_cast<int>(blockIdx.x) >= a.P) {
     finish_share<G, TW, PAIR, OUTF32, ONE>(a, static_cast<int>(blockIdx.x) - a.P);
     return;
