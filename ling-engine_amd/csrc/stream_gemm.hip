@@ -1123,10 +1123,11 @@ __global__ void __launch_bounds__(256) rmsnorm_half_reg_kernel(const float* __re
   if (tid == 0) xinv[r] = ldexpf(1.f, e - 15);
 }
 
-// The same for rows of whole 8-value pieces at 16-byte aligned pointers, laid out over the threads as in
-// half_rows_vec_kernel. The squares of a thread's pieces are added in order, then the lanes, then the waves in order.
-// (5 x 5120, inputs not in a cache: 10.2 -> 4.4 us.)
-template <int NV>
+// The same for rows of whole 8-value pieces, laid out over the threads as in half_rows_vec_kernel. The squares of a thread's
+// pieces are added in order, then the lanes, then the waves in order. (5 x 5120, inputs not in a cache: 10.2 -> 4.4 us.)
+// ALIGNED: every pointer at 16 bytes. The other form takes the same values value by value, so that where a caller's
+// buffers lie changes no bit of its result.
+template <int NV, bool ALIGNED>
 __global__ void __launch_bounds__(1024) rmsnorm_half_vec_kernel(const float* __restrict__ x, const uint16_t* __restrict__ w,
                                                                 float* __restrict__ out, _Float16* __restrict__ xh,
                                                                 float* __restrict__ xinv, int H, float eps, bool gemma) {
@@ -1137,8 +1138,16 @@ __global__ void __launch_bounds__(1024) rmsnorm_half_vec_kernel(const float* __r
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
     const int p = min(static_cast<int>(threadIdx.x) + T * j, pieces - 1);
-    load8(x + r * H + 8 * p, v[j]);
-    load8(w + 8 * p, wf[j]);
+    if constexpr (ALIGNED) {
+      load8(x + r * H + 8 * p, v[j]);
+      load8(w + 8 * p, wf[j]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        v[j][i] = x[r * H + 8 * p + i];
+        wf[j][i] = bf16_to_f32(w[8 * p + i]);
+      }
+    }
   }
   float ss = 0.f;
 #pragma unroll
@@ -1163,9 +1172,14 @@ __global__ void __launch_bounds__(1024) rmsnorm_half_vec_kernel(const float* __r
     }
     const int p = static_cast<int>(threadIdx.x) + T * j;
     if (p < pieces) {
-      f32x4* o = reinterpret_cast<f32x4*>(out + r * H + 8 * p);
-      o[0] = f32x4{v[j][0], v[j][1], v[j][2], v[j][3]};
-      o[1] = f32x4{v[j][4], v[j][5], v[j][6], v[j][7]};
+      float* const o = out + r * H + 8 * p;
+      if constexpr (ALIGNED) {
+        reinterpret_cast<f32x4*>(o)[0] = f32x4{v[j][0], v[j][1], v[j][2], v[j][3]};
+        reinterpret_cast<f32x4*>(o)[1] = f32x4{v[j][4], v[j][5], v[j][6], v[j][7]};
+      } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) o[i] = v[j][i];
+      }
     }
   }
   mx = workgroup_max(mx, redmax);
@@ -1175,7 +1189,14 @@ __global__ void __launch_bounds__(1024) rmsnorm_half_vec_kernel(const float* __r
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
     const int p = static_cast<int>(threadIdx.x) + T * j;
-    if (p < pieces) *reinterpret_cast<u32x4*>(xh + r * H + 8 * p) = to_half8(v[j], sc);
+    if (p < pieces) {
+      if constexpr (ALIGNED) {
+        *reinterpret_cast<u32x4*>(xh + r * H + 8 * p) = to_half8(v[j], sc);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) xh[r * H + 8 * p + i] = static_cast<_Float16>(v[j][i] * sc);
+      }
+    }
   }
   if (threadIdx.x == 0) xinv[r] = ldexpf(1.f, e - 15);
 }
@@ -1497,12 +1518,12 @@ int check_rows(const char* name, int M, int N, int K) {
   return LQ_OK;
 }
 
-// Whether rows of K values can be taken in 8-value pieces with 16-byte accesses, and the threads of a row's workgroup for
-// NV pieces per thread (the fewest waves that cover it).
-bool row_pieces(int K, const void* a, const void* b, const void* c = nullptr, const void* d = nullptr) {
-  const uintptr_t bits = reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b) | reinterpret_cast<uintptr_t>(c) |
-                         reinterpret_cast<uintptr_t>(d);
-  return K % 8 == 0 && K <= 32768 && bits % 16 == 0;
+// Whether rows of K values are taken in 8-value pieces, whether with 16-byte accesses, and the threads of a row's workgroup
+// for NV pieces per thread (the fewest waves that cover it).
+bool row_pieces(int K) { return K % 8 == 0 && K <= 32768; }
+bool aligned16(const void* a, const void* b, const void* c = nullptr, const void* d = nullptr) {
+  return ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b) | reinterpret_cast<uintptr_t>(c) |
+           reinterpret_cast<uintptr_t>(d)) % 16) == 0;
 }
 int row_threads(int K, int nv) { return 64 * cdiv(cdiv(K / 8, nv), 64); }
 
@@ -1512,7 +1533,7 @@ int half_rows(bool bf16in, const void* x, int M, int K, uint16_t* xh, float* xin
   if (!x || !xh || !xinv) return fail(LQ_ERR_ARG, std::string(nm) + ": null pointer");
   // rows of up to 32768 values: one block per row, the row in registers, in 16-byte pieces where the row and the pointers
   // allow them
-  if (row_pieces(K, x, xh)) {
+  if (row_pieces(K) && aligned16(x, xh)) {
     auto vec = [&](auto nv, auto in) {
       constexpr int NV = decltype(nv)::value;
       using InT = decltype(in);
@@ -1648,13 +1669,19 @@ int lq_rmsnorm_half(const float* x, const uint16_t* w, float* out, uint16_t* xh,
   if (!x || !w || !out || !xh || !xinv) return fail(LQ_ERR_ARG, "rmsnorm_half: null pointer");
   const hipStream_t s = static_cast<hipStream_t>(stream);
   _Float16* const xh16 = reinterpret_cast<_Float16*>(xh);
-  // rows of up to 32768 values in 16-byte pieces where they and the pointers allow it, else of up to 8192: the row and its
-  // weights in registers
-  if (row_pieces(H, x, w, out, xh)) {
+  // rows of up to 32768 values in 8-value pieces where they are whole ones, else of up to 8192: the row and its weights in
+  // registers. Which is a matter of H alone: the forms add a row's squares in different orders.
+  if (row_pieces(H)) {
+    const bool aligned = aligned16(x, w, out, xh);
     auto vec = [&](auto nv) {
       constexpr int NV = decltype(nv)::value;
-      hipLaunchKernelGGL(rmsnorm_half_vec_kernel<NV>, dim3(rows), dim3(row_threads(H, NV)), 0, s, x, w, out, xh16, xinv, H,
-                         eps, gemma != 0);
+      const dim3 threads(row_threads(H, NV));
+      if (aligned)
+        hipLaunchKernelGGL((rmsnorm_half_vec_kernel<NV, true>), dim3(rows), threads, 0, s, x, w, out, xh16, xinv, H, eps,
+                           gemma != 0);
+      else
+        hipLaunchKernelGGL((rmsnorm_half_vec_kernel<NV, false>), dim3(rows), threads, 0, s, x, w, out, xh16, xinv, H, eps,
+                           gemma != 0);
     };
     if (H <= 8192) vec(std::integral_constant<int, 1>{});
     else if (H <= 16384) vec(std::integral_constant<int, 2>{});

@@ -229,6 +229,23 @@ def test_rmsnorm_half(L, rows, H, gemma):
     assert np.array_equal(xinv.cpu().numpy(), ci)
 
 
+@pytest.mark.parametrize("rows,H", [(5, 5120), (9, 8200), (9, 20480)])
+def test_rmsnorm_half_bits_do_not_depend_on_alignment(L, rows, H):
+    """Buffers at any element's address give the bits of buffers at 16 bytes: the sum of squares has one order."""
+    x = to_dev(O.normal_f32(82 + rows, 2.0, (rows, H)))
+    w = bf16_dev(O.normal_bf16(83 + rows, 0.1, (H,)))
+    want = [t.clone() for t in L.rmsnorm_half(x, w, 1e-6)]
+
+    def moved(t, by):
+        m = torch.empty(t.numel() + by, dtype=t.dtype, device=DEV)[by:].view(t.shape)
+        return m.copy_(t)
+
+    for bx, bw in ((1, 0), (0, 1), (3, 5)):
+        got = L.rmsnorm_half(moved(x, bx), moved(w, bw), 1e-6)
+        for g, r, name in zip(got, want, ("out", "xh", "xinv")):
+            assert torch.equal(g, r), f"{name}: x {bx}, w {bw} elements on"
+
+
 # ---------------- activation producers (reference prefill_gemm.cu:382-459, 607-637) ----------------
 def _reference_test_activations(M, K, seed):
     """The reference's own test distribution (tests/prefill_tests.cu:58-60): N(0, 1) * 0.003, every 97th value
