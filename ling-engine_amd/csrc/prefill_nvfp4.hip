@@ -12,13 +12,14 @@
 // accumulation across all of K; alpha is applied at the end.
 //
 //  * A wave computes 128 weight rows x 64 tokens (8 x 4 MFMA tiles, 128 accumulator registers; SwiGLU: 64 gate rows and
-//    the same 64 up rows; NI = 4: 64 rows, for calls with few tiles). Per 128-value chunk a lane holds the raw 16 bytes (32 E2M1 values) and the 2 scales of its
-//    row for each of its 8 weight tiles and 4 token tiles, and dequantizes one 8-value step at a time: lane (r, t)
-//    supplies K 32t + 8s .. +8 at step s for both operands (a permutation of K inside the chunk, harmless as both
-//    operands use it; the weights' tiled layout holds exactly these 16 bytes per (row, t), slot r * 4 + t).
-//  * The 8 waves of a workgroup are WM along the tokens x WK = 8 / WM along K, so a tile is 64 WM tokens high and a prompt
-//    of a few hundred tokens still gives every CU two waves per SIMD, at the wave tile's ratio of dequantization to
-//    MFMAs. Wave k of a K group takes chunks k, k + WK, ..; the group's FP32 sums meet in LDS at the end and are added
+//    the same 64 up rows; NI = 4: 64 rows, for calls with few tiles). Per 128-value chunk a lane holds the raw 16 bytes
+//    (32 E2M1 values) and the 2 scales of its row for each of its 8 weight tiles and 4 token tiles, and dequantizes one
+//    8-value step at a time: lane (r, t) supplies K 32t + 8s .. +8 at step s for both operands (a permutation of K
+//    inside the chunk, harmless as both operands use it; the weights' tiled layout holds exactly these 16 bytes per
+//    (row, t), slot r * 4 + t).
+//  * The 8 waves of a workgroup are WM (1 or 2) along the tokens x WK = 8 / WM along K, so a tile is 64 WM tokens high and a
+//    prompt of a few hundred tokens still gives every CU two waves per SIMD, at the wave tile's ratio of dequantization
+//    to MFMAs. Wave k of a K group takes chunks k, k + WK, ..; the group's FP32 sums meet in LDS at the end and are added
 //    in wave order.
 //  * Nothing is shared while a wave computes, so there are no barriers: each wave streams its own operands to its own
 //    13.5 KB of LDS by direct loads, takes a landed chunk into registers (60 of them) and at once has the next one loaded
@@ -29,7 +30,7 @@
 //
 // What bounds it: the dequantization and the MFMAs share the SIMD's issue (3 VALU instructions per MFMA). Tiles of 256 x
 // 256 over 8 waves, which read a step's word from LDS just ahead of its use, took 430 us at 300 x 5120 x 17408 (40 tiles
-// on 256 CUs), 447 at 2048 x 5120 x 17408 and 760 for SwiGLU at 2048 x 17408 x 5120: now 60, 318 and 637.
+// on 256 CUs), 447 at 2048 x 5120 x 17408 and 760 for SwiGLU at 2048 x 17408 x 5120: now 63, 312 and 637.
 #include "lq_common.hpp"
 
 #include <string>
@@ -289,34 +290,32 @@ int tile_launch(Nvfp4Args a, const char* name, hipStream_t s) {
   return check_launch(name);
 }
 
-// The tile, by an estimate of the time: rounds of one tile per CU, each of which takes every wave of a K group through its
-// share of the chunks and then the sums. A higher tile reads its weights fewer times and its chunk costs a little less, a
-// lower one leaves fewer CUs idle and pads fewer tokens; half the weight rows (NI = 4) dequantize more per MFMA, and pay
-// where whole wave tiles would leave half the CUs without work. Measured (us at WM = 1, 2, 4 with NI = 8, then NI = 4):
-// 100 x 5120 x 5120 21, 34, 60, 14; 200 x 2048 x 4096 18, 29, 50, 12; 160 x 5120 x 17408 56, 99, 186, 42; 200 x 5120 x
-// 5120 23, 35, 61, 26; 300 x 5120 x 17408 59, 100, 188, 74; 500 x 17408 x 5120 114, 116, 133; 2048 x 5120 x 17408 321, 340,
-// 412; 4096 x 7168 x 5120 294, 264, 275; SwiGLU 2048 x 17408 x 5120 721, 650, 637 and 1000 x 3072 x 1024 27, 26, 21. The
-// estimate is within 15 % of these. (WM = 8, no K split: 262 at 4096 x 7168 x 5120, slower elsewhere; NI = 4 with WM = 2
-// never ahead by more than 2 %.)
+// The tile. How many waves share K (8 / wm) is a matter of the matrix alone: the FP32 sums are then taken in one order
+// whatever the number of tokens, and a row's result has the same bits in every call. Eight waves leave the fewest CUs idle,
+// four pay a K group's closing sums half as often; four are taken where the matrix' own tiles (128 weight rows) are at least
+// half the CUs. Measured, us, eight and four (M = 128, 512, 2048, 4096): SwiGLU 17408 x 5120 70 81, 201 188, 719 637, 1409
+// 1280 and 9728 x 2560 30 26, 71 67, 257 215, 506 407; N = 34816, K = 5120 69 81, 201 187 (M = 500), 730 657, 1439 1297. On the
+// other side of the line SwiGLU 6144 x 2048 14 20, 37 38, 140 115, 274 239; N = 7168, K = 5120 22 35, 45 40 (M = 500), 162
+// 151, 309 274; N = 5120, K = 17408 58 106, 111 103 (M = 500), 312 325, 628 591. (Chosen by M as well, with two waves along K
+// among the choices, 1-16 % less over M = 81 .. 4096 at one matrix, most of it at 1500 tokens and more and short K: not
+// worth results that depend on how a prompt is cut.)
+//
+// With eight waves along K, half the weight rows (NI = 4; the same sums) dequantize more per MFMA, and pay where whole wave
+// tiles would leave half the CUs without work: by an estimate of the time, rounds of one tile per CU, each of which takes
+// every wave through its share of the chunks and then the sums (NI = 8, NI = 4: 128 x 5120 x 5120 22.1, 15.3; 300 x 5120 x
+// 5120 24.3, 27.6; 128 x 5120 x 17408 58, 42; 500 x 2048 x 4096 19.4, 13.9). NI = 4 with four waves never was ahead by more than 2 %.
 struct TileKind {
   int ni, wm;
-  double chunk, tile;  // microseconds
 };
-constexpr TileKind kKinds[] = {{8, 1, 3.45, 5.}, {8, 2, 3.2, 5.}, {8, 4, 3.2, 6.}, {4, 1, 2.15, 4.}};
 
 TileKind choose_tile(bool swiglu, int M, int N, int C, long long cus) {
-  TileKind best = kKinds[0];
-  double best_us = 0.;
-  for (const TileKind& k : kKinds) {
-    if (swiglu && k.ni != 8) continue;
-    const long long tiles = static_cast<long long>(N / (swiglu ? 64 : 16 * k.ni)) * cdiv(M, 64 * k.wm);
-    const double us = static_cast<double>((tiles + cus - 1) / cus) * (cdiv(C, 8 / k.wm) * k.chunk + k.tile);
-    if (&k == kKinds || us < best_us) {
-      best_us = us;
-      best = k;
-    }
-  }
-  return best;
+  if (2LL * (N / (swiglu ? 64 : 128)) >= cus) return {8, 2};
+  if (swiglu) return {8, 1};
+  auto us = [&](int ni, double chunk, double tile) {
+    const long long tiles = static_cast<long long>(N / (16 * ni)) * cdiv(M, 64);
+    return static_cast<double>((tiles + cus - 1) / cus) * (cdiv(C, 8) * chunk + tile);
+  };
+  return us(4, 2.15, 4.) < us(8, 3.45, 5.) ? TileKind{4, 1} : TileKind{8, 1};
 }
 
 template <bool SWIGLU>
@@ -338,11 +337,7 @@ int nvfp4_launch(Nvfp4Args a, const char* name, hipStream_t s) {
   const TileKind k = choose_tile(SWIGLU, a.M, a.N, a.C, device_cus(dev));
   if constexpr (!SWIGLU)
     if (k.ni == 4) return tile_launch<SWIGLU, 4, 1>(a, name, s);
-  switch (k.wm) {
-    case 1: return tile_launch<SWIGLU, 8, 1>(a, name, s);
-    case 2: return tile_launch<SWIGLU, 8, 2>(a, name, s);
-    default: return tile_launch<SWIGLU, 8, 4>(a, name, s);
-  }
+  return k.wm == 1 ? tile_launch<SWIGLU, 8, 1>(a, name, s) : tile_launch<SWIGLU, 8, 2>(a, name, s);
 }
 
 }  // namespace
@@ -351,6 +346,12 @@ int nvfp4_launch(Nvfp4Args a, const char* name, hipStream_t s) {
 using namespace lq;
 
 extern "C" {
+
+// Test hook (not part of the interface): the tile of a product on `cus` CUs, 16 * NI + WM.
+int lq_debug_prefill_nvfp4_tile(int swiglu, int M, int N, int K, int cus) {
+  const TileKind k = choose_tile(swiglu != 0, M, N, K / 128, cus);
+  return 16 * k.ni + k.wm;
+}
 
 int lq_prefill_gemm_nvfp4(const uint8_t* xq, const uint8_t* xs, int M, const uint8_t* w, float alpha, float* y, int ldy,
                           int N, int K, int accumulate, void* stream, const uint8_t* wsf) {

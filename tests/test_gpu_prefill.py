@@ -395,6 +395,30 @@ def test_prefill_nvfp4_tiles(L, M, N, K):
     assert (q != rq).float().mean().item() <= 3e-3 and (sf != rsf).float().mean().item() <= 1e-3
 
 
+# matrices with eight waves along K (in both weight tiles of the plain form) and with four, remainders of chunks
+@pytest.mark.parametrize("N,K", [(384, 1408), (6528, 1152), (16384, 1152)])
+def test_prefill_nvfp4_rows_do_not_depend_on_m(L, N, K):
+    """A row's result has the same bits in a call of any number of tokens, plain and SwiGLU. (Block scales over a range of
+    2^9 in both operands: the FP32 sums are not exact, so another order of them shows.)"""
+    M = 1030
+    rng = np.random.default_rng(170 + N)
+
+    def codes_and_scales(rows):
+        return (to_dev(rng.integers(0, 256, (rows, K // 2), dtype=np.uint8)),
+                to_dev(rng.integers(0x20, 0x68, (rows, K // 16), dtype=np.uint8)))
+
+    raw = L.retile_nvfp4(*codes_and_scales(N))
+    xq, xs = codes_and_scales(M)
+    alpha = float(1.0 / L.prefill_gemm_nvfp4(xq, xs, raw, 1.0, N).std())
+    y = L.prefill_gemm_nvfp4(xq, xs, raw, alpha, N)
+    q, sf = L.prefill_swiglu_nvfp4(xq, xs, raw, alpha, raw, alpha, N, 0.05)
+    for m in (1, 64, 65, 260, 700):
+        ym = L.prefill_gemm_nvfp4(xq[:m], xs[:m], raw, alpha, N)
+        assert torch.equal(ym.view(torch.int32), y[:m].view(torch.int32)), f"{m} of {M} rows"
+        qm, sfm = L.prefill_swiglu_nvfp4(xq[:m], xs[:m], raw, alpha, raw, alpha, N, 0.05)
+        assert torch.equal(qm, q[:m]) and torch.equal(sfm, sf[:m]), f"SwiGLU, {m} of {M} rows"
+
+
 def test_prefill_nvfp4_device_quantized_activations(L):
     """The activations from quant_act_nvfp4 on the GPU, a larger shape, every 16th row checked."""
     M, N, K = 1024, 2048, 2048
