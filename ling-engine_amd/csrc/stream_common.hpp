@@ -113,9 +113,14 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base) {
 }
 constexpr int kNT = 2;  // slc: streaming (non-temporal) weights
 
-template <int WF, int T>
+// Whether a kernel takes its NVFP4 scale bytes through LDS (load_scales, below) or each lane its own with the weights.
+template <int G, int WF, bool CVT>
+constexpr bool kLdsScales = WF == kFp4Coded || (WF == kFp4 && (CVT || G != 2));
+
+// scale_off: where each lane loads its own scale pairs (raw NVFP4 without kLdsScales), the lane's offset to them.
+template <int WF, int T, bool OWN_SCALES = false>
 __device__ __forceinline__ void load_w(WRegs<WF, T>& R, const __amdgpu_buffer_rsrc_t (&rs)[T], const int (&toff)[T],
-                                       int c, int lane_off) {
+                                       int c, int lane_off, int scale_off = 0) {
 #pragma unroll
   for (int i = 0; i < T; ++i) {
     if constexpr (WF == kFp8) {
@@ -125,6 +130,8 @@ __device__ __forceinline__ void load_w(WRegs<WF, T>& R, const __amdgpu_buffer_rs
     } else {
       const int so = toff[i] + c * (WF == kFp4 ? kTileBytesFp4 : kValueBytesFp4);
       R.v[i][0] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs[i], lane_off, so, kNT));
+      if constexpr (OWN_SCALES)
+        R.sc[i] = static_cast<uint16_t>(__builtin_amdgcn_raw_buffer_load_b16(rs[i], scale_off, so, 0));
     }
   }
 }
@@ -133,7 +140,9 @@ __device__ __forceinline__ void load_w(WRegs<WF, T>& R, const __amdgpu_buffer_rs
 // 16 pieces of raw scales, 12 of codes), which go through the wave's 512 bytes of LDS to the lanes that use them. They are
 // loaded and stored with the chunk's activations, a chunk ahead of their use. (Loaded by the lanes that use them they were
 // four 2-byte loads per chunk, coded eight of one byte, on the path that the weight stream shares: coded 17408 x 5120 at
-// M = 1 20.4 -> 18.5 us, 5120 x 25600 at M = 16 25.6 -> 22.5; raw 16.8 -> 16.5 and 20.4 -> 20.0 at M = 16.)
+// M = 1 20.4 -> 18.5 us, 5120 x 25600 at M = 16 25.6 -> 22.5; raw 16.8 -> 16.5 and 20.4 -> 20.0 at M = 16. Raw scales
+// beside an FP16 row copy of 17 to 32 rows stay with the lanes:
+// 5120 x 25600 at M = 17, 24, 32 25.5, 25.8, 25.9 us, through LDS 26.3, 26.7, 26.8; 17408 x 5120 22.0, 22.2, 23.2 and 22.4, 22.7, 23.7.)
 __device__ __forceinline__ u32x2 load_scales(const __amdgpu_buffer_rsrc_t& rs, int soff, int lane_off, unsigned oob) {
   return __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rs, static_cast<int>(lane_off | oob), soff, 0));
 }
@@ -706,8 +715,8 @@ template <int G>
 struct SmemFp4 : Smem<G> {
   alignas(16) uint8_t sc[Smem<G>::NSLOT][4][512];  // a chunk's scale bytes, each wave its own
 };
-template <int G, int WF>
-using StreamSmem = std::conditional_t<WF == kFp8, Smem<G>, SmemFp4<G>>;
+template <int G, int WF, bool CVT>
+using StreamSmem = std::conditional_t<kLdsScales<G, WF, CVT>, SmemFp4<G>, Smem<G>>;
 
 // Body modes: kYCoh = the pair epilogue's stores write through (a later phase of the same launch reads them);
 // kXCoh = activations are read agent-coherently and only after `ready()` returns (the weight ring's first

@@ -64,8 +64,8 @@ namespace {
 // wave 0's weights in xpre.
 template <int G, int WF, int TW, bool F16, bool PAIR, bool OUTF32, int MODE, bool ONE = false, int NPRE = 0,
           class Ready>
-__device__ __forceinline__ void stream_body(const StreamArgs& a, int p, StreamSmem<G, WF>& sm, Ready&& ready,
-                                            uint8_t* xpre = nullptr) {
+__device__ __forceinline__ void stream_body(const StreamArgs& a, int p, StreamSmem<G, WF, (MODE & kCvt) != 0>& sm,
+                                            Ready&& ready, uint8_t* xpre = nullptr) {
   constexpr int T = TW;
   constexpr int PF = pf_stages<T>(G);
   constexpr bool BPRE = Smem<G>::BPRE;
@@ -73,6 +73,7 @@ __device__ __forceinline__ void stream_body(const StreamArgs& a, int p, StreamSm
   constexpr bool YCOH = (MODE & kYCoh) != 0, XCOH = (MODE & kXCoh) != 0;
   constexpr int XPOL = XCOH ? kSc1 : 0;
   constexpr bool CVT = (MODE & kCvt) != 0;
+  constexpr bool LDS_SC = kLdsScales<G, WF, CVT>, OWN_SC = WF == kFp4 && !LDS_SC;
   static_assert(!CVT || F16, "converted activations feed the FP16 MFMA");
   static_assert(!BPRE || PF >= 3, "the operand prefetch needs a chunk of lookahead");
   static_assert(NPRE == 0 || (XCOH && !CVT), "run-ahead chunks are for the activation-waiting form");
@@ -131,6 +132,7 @@ __device__ __forceinline__ void stream_body(const StreamArgs& a, int p, StreamSm
   // weight lane offset: FP8 piece ((h*2 + 0)*8 + g)*4 + t (q = 1 is 512 bytes on); NVFP4 slot r*4 + t
   const int slot = r * 4 + t;
   const int lane_off = WF == kFp8 ? (((r >> 3) * 16 + (r & 7)) * 4 + t) * 16 : slot * 16;
+  const int scale_off = kValueBytesFp4 + 2 * slot;  // OWN_SC: the lane's scale pair of a raw NVFP4 block
 
   // The workgroup's units form one continuous stream through the register ring, across tile-group
   // boundaries: the load cursor (ltg, lc) runs PF - 1 chunks ahead of the compute cursor (ctg, cc).
@@ -143,12 +145,12 @@ __device__ __forceinline__ void stream_body(const StreamArgs& a, int p, StreamSm
 
   WRegs<WF, T> wr[PF];
   u32x4 xr[PF][G];
-  u32x2 scr[PF];  // NVFP4: the lane's piece of the stage's scale bytes
+  u32x2 scr[PF];  // LDS_SC: the lane's piece of the stage's scale bytes
   // Every ring load is issued unconditionally (the wait counts then hold on every path); a load past the
   // stream's end is turned into an out-of-range buffer load (offset >= num_records), which returns zeros and
   // touches no memory.
   auto load_x = [&](int j, int lcj, unsigned oob) {
-    if constexpr (WF != kFp8)
+    if constexpr (LDS_SC)
       scr[j] = load_scales(L.rs[0], L.soff + lcj * (WF == kFp4 ? kTileBytesFp4 : kCodeBytesFp4), L.slane, oob);
 #pragma unroll
     for (int i = 0; i < G; ++i)
@@ -172,7 +174,7 @@ __device__ __forceinline__ void stream_body(const StreamArgs& a, int p, StreamSm
     __builtin_amdgcn_sched_barrier(0);
     load_x(j, lc, oob);
     __builtin_amdgcn_sched_barrier(0);
-    load_w<WF, T>(wr[j], L.rs, L.toff, lc, static_cast<int>(lane_off | oob));
+    load_w<WF, T, OWN_SC>(wr[j], L.rs, L.toff, lc, static_cast<int>(lane_off | oob), static_cast<int>(scale_off | oob));
     __builtin_amdgcn_sched_barrier(0);
     advance();
   };
@@ -189,12 +191,13 @@ __device__ __forceinline__ void stream_body(const StreamArgs& a, int p, StreamSm
   };
   auto load_stage_w = [&](int j) {
     __builtin_amdgcn_sched_barrier(0);
-    load_w<WF, T>(wr[j], L.rs, L.toff, lc, static_cast<int>(lane_off | stage_oob));
+    load_w<WF, T, OWN_SC>(wr[j], L.rs, L.toff, lc, static_cast<int>(lane_off | stage_oob),
+                          static_cast<int>(scale_off | stage_oob));
     __builtin_amdgcn_sched_barrier(0);
     advance();
   };
   auto put_x = [&](int j, int sl) {
-    if constexpr (WF != kFp8) *reinterpret_cast<u32x2*>(sm.sc[sl][wave] + lane * 8) = scr[j];
+    if constexpr (LDS_SC) *reinterpret_cast<u32x2*>(sm.sc[sl][wave] + lane * 8) = scr[j];
 #pragma unroll
     for (int i = 0; i < G; ++i) {
       if constexpr (CVT) {
@@ -206,12 +209,12 @@ __device__ __forceinline__ void stream_body(const StreamArgs& a, int p, StreamSm
     }
   };
   auto scales = [&](uint32_t (&sc)[T], int sl) {
-    if constexpr (WF != kFp8)
+    if constexpr (LDS_SC)
 #pragma unroll
       for (int i = 0; i < T; ++i) sc[i] = read_scales<WF>(sm.sc[sl][wave], i, slot);
   };
   auto take_scales = [&](WRegs<WF, T>& R, const uint32_t (&sc)[T]) {
-    if constexpr (WF != kFp8)
+    if constexpr (LDS_SC)
 #pragma unroll
       for (int i = 0; i < T; ++i) R.sc[i] = sc[i];
   };
@@ -438,7 +441,7 @@ __device__ __forceinline__ void stream_body(const StreamArgs& a, int p, StreamSm
 #pragma unroll
           for (int g = 0; g < G; ++g) scc[g] = scn[g];
         }
-        if constexpr (WF != kFp8) {
+        if constexpr (LDS_SC) {
 #pragma unroll
           for (int i = 0; i < T; ++i) wsc[i] = wsn[i];
         }
@@ -566,7 +569,7 @@ __device__ __forceinline__ void stream_body(const StreamArgs& a, int p, StreamSm
 
 template <int G, int WF, int TW, bool F16, bool PAIR, bool OUTF32, bool CVT = false, bool ONE = false>
 __global__ void __launch_bounds__(kThreads) stream_kernel(const StreamArgs a) {
-  __shared__ __attribute__((aligned(16))) StreamSmem<G, WF> sm;
+  __shared__ __attribute__((aligned(16))) StreamSmem<G, WF, CVT> sm;
   if (static_cast<int>(blockIdx.x) >= a.P) {
     finish_share<G, TW, PAIR, OUTF32, ONE>(a, static_cast<int>(blockIdx.x) - a.P);
     return;
