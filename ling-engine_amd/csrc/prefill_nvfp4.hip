@@ -290,32 +290,35 @@ int tile_launch(Nvfp4Args a, const char* name, hipStream_t s) {
   return check_launch(name);
 }
 
-// The tile. How many waves share K (8 / wm) is a matter of the matrix alone: the FP32 sums are then taken in one order
-// whatever the number of tokens, and a row's result has the same bits in every call. Eight waves leave the fewest CUs idle,
-// four pay a K group's closing sums half as often; four are taken where the matrix' own tiles (128 weight rows) are at least
-// half the CUs. Measured, us, eight and four (M = 128, 512, 2048, 4096): SwiGLU 17408 x 5120 70 81, 201 188, 719 637, 1409
-// 1280 and 9728 x 2560 30 26, 71 67, 257 215, 506 407; N = 34816, K = 5120 69 81, 201 187 (M = 500), 730 657, 1439 1297. On the
-// other side of the line SwiGLU 6144 x 2048 14 20, 37 38, 140 115, 274 239; N = 7168, K = 5120 22 35, 45 40 (M = 500), 162
-// 151, 309 274; N = 5120, K = 17408 58 106, 111 103 (M = 500), 312 325, 628 591. (Chosen by M as well, with two waves along K
-// among the choices, 1-16 % less over M = 81 .. 4096 at one matrix, most of it at 1500 tokens and more and short K: not
-// worth results that depend on how a prompt is cut.)
+// The tile, by an estimate of the time: rounds of one tile per CU, each of which takes every wave through its share of the
+// chunks and then the sums. A wave tile of half the weight rows (NI = 4) dequantizes more per MFMA, and pays where whole ones
+// leave half the CUs without work (us at NI = 8 and 4, WM = 1: 128 x 5120 x 5120 22.1, 15.3; 300 x 5120 x 5120 24.3, 27.6;
+// 128 x 5120 x 17408 58, 42; 500 x 2048 x 4096 19.4, 13.9).
 //
-// With eight waves along K, half the weight rows (NI = 4; the same sums) dequantize more per MFMA, and pay where whole wave
-// tiles would leave half the CUs without work: by an estimate of the time, rounds of one tile per CU, each of which takes
-// every wave through its share of the chunks and then the sums (NI = 8, NI = 4: 128 x 5120 x 5120 22.1, 15.3; 300 x 5120 x
-// 5120 24.3, 27.6; 128 x 5120 x 17408 58, 42; 500 x 2048 x 4096 19.4, 13.9). NI = 4 with four waves never was ahead by more than 2 %.
+// How many waves share K (8 / WM) is a matter of the matrix alone: the FP32 sums are then taken in one order whatever the
+// number of tokens, and a row's result has the same bits in every call. Eight waves leave the fewest CUs idle, four pay a
+// tile's closing sums half as often; taken is what is faster over prompts of 128 to 4096 tokens, by the product of the
+// ratios. Measured at M = 128, 512, 2048, 4096, eight and four: SwiGLU 17408 x 5120 70 81, 201 188, 719 637, 1409 1280;
+// 6144 x 2048 14 20, 37 38, 140 115, 274 239 and N = 34816, K = 5120 69 81, 201 187 (M = 500), 730 657, 1439 1297 (four);
+// SwiGLU 5120 x 5120 26 40, 66 74, 221 194, 425 394; N = 7168, K = 5120 16 35, 45 40 (M = 500), 162 151, 309 274 and N = 5120,
+// K = 17408 42 106, 111 103 (M = 500), 312 325, 628 591 (eight). Over 33 matrices and M = 81 .. 4096 the rule is 5 % from
+// the faster of the two at each M. (Two waves along K at M >= 1500 and short K: up to 20 % less than eight, not worth
+// results that depend on how a prompt is cut. NI = 4 with WM = 2 was never ahead by more than 2 %.)
 struct TileKind {
   int ni, wm;
+  double chunk, tile;  // microseconds
 };
+constexpr TileKind kWhole{8, 1, 3.45, 5.}, kHalf{4, 1, 2.15, 4.}, kFour{8, 2, 3.2, 5.};
 
 TileKind choose_tile(bool swiglu, int M, int N, int C, long long cus) {
-  if (2LL * (N / (swiglu ? 64 : 128)) >= cus) return {8, 2};
-  if (swiglu) return {8, 1};
-  auto us = [&](int ni, double chunk, double tile) {
-    const long long tiles = static_cast<long long>(N / (16 * ni)) * cdiv(M, 64);
-    return static_cast<double>((tiles + cus - 1) / cus) * (cdiv(C, 8) * chunk + tile);
+  auto us = [&](const TileKind& k, int m) {
+    const long long tiles = static_cast<long long>(N / (swiglu ? 64 : 16 * k.ni)) * cdiv(m, 64 * k.wm);
+    return static_cast<double>((tiles + cus - 1) / cus) * (cdiv(C, 8 / k.wm) * k.chunk + k.tile);
   };
-  return us(4, 2.15, 4.) < us(8, 3.45, 5.) ? TileKind{4, 1} : TileKind{8, 1};
+  auto eight = [&](int m) { return !swiglu && us(kHalf, m) < us(kWhole, m) ? kHalf : kWhole; };
+  double ratio = 1.;
+  for (int m = 128; m <= 4096; m *= 2) ratio *= us(eight(m), m) / us(kFour, m);
+  return ratio > 1. ? kFour : eight(M);
 }
 
 template <bool SWIGLU>
