@@ -23,6 +23,9 @@
 //  * Tile order: each XCD works through a contiguous range of a grouped raster (kGroupN weight tiles x every
 //    token tile per group), so the workgroups running at once on an XCD share the K slices of both operands
 //    in its L2 instead of re-streaming the whole activation matrix per weight tile.
+//  * That is prefill_fp8_kernel, for products of many tiles (a last round of few tiles is split along K, the parts
+//    exchanged as FP32 partials). prefill_tile_kernel computes products whose 256 x 256 tiles would leave CUs without
+//    work, in tiles of 64 x 64 to 128 x 128 with two to four LDS stages; choose_tile picks.
 #include "lq_common.hpp"
 #include "lq_prefill_offsets.hpp"
 #include "lq_workspace.hpp"
@@ -255,7 +258,7 @@ __global__ void __launch_bounds__(kThreads) prefill_fp8_kernel(const PrefillArgs
       __builtin_amdgcn_s_setprio(1);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        // (scales 0: the compiler takes the unscaled instruction, which needs no scale load before it, 2 % faster)
+        // (scales that are the constant 0 select the unscaled instruction, which needs no scale load before it: 2 % faster)
         if constexpr (BLOCK)
           pr[j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(af, bf[j], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 0,
                                                                   0, 0);
@@ -637,11 +640,15 @@ int tile_launch(PrefillArgs a, const char* name, hipStream_t s) {
 // less each output costs, but tiles come in whole numbers per CU, so a product with few of them is done sooner in
 // smaller ones. A launch costs 4 us; a split last round of 256 x 256 tiles 10 us more and 0.07 us per part, for the
 // exchange. The smallest sum wins, the 256 x 256 tile unless another is 5 % better. Measured, block-scaled (M x N x K,
-// us, rotating over 600 MB of weights): 100 x 5120 x 5120 35 -> 15 (64 x 64), 200 x 7168 x 5120 40 -> 21 (128 x 64),
-// 300 x 5120 x 17408 86 -> 70 (128 x 64), 512 x 5120 x 5120 42 -> 31 (128 x 128), 500 x 17408 x 5120 83 -> 80
-// (128 x 128 x2); 1000 x 5120 x 17408 stays at 110 (132 in 128 x 128 x2). 64 x 128 (15 % faster at 300 x 5120 x 17408,
-// 10 % slower elsewhere) and 128 x 256 (7 % faster at 777 x 5120 x 6144, 9 % slower at 256 x 17408 x 5120) were not
-// worth their kernels.
+// us, rotating over 500 MB of weights): 200 x 2048 x 4096 32 -> 12 (64 x 64), 200 x 7168 x 5120 42 -> 22 (128 x 64),
+// 300 x 5120 x 17408 83 -> 72 (128 x 64), 512 x 5120 x 5120 45 -> 34 (128 x 128), 1500 x 5120 x 17408 238 -> 153 (128 x 128
+// x2); 1000 x 5120 x 17408 stays at 114 (133 in 128 x 128 x2) and 500 x 17408 x 5120 at 83 (80 in 128 x 128 x2).
+//
+// The constants are the block-scaled form's. The estimates are 0.8-1.3 of what was measured (per tensor, which has no
+// folds, 0.6-1.1), but the order is what counts: over nine matrices and M = 200 .. 4096 the tile taken is on average 1.0 %
+// (per tensor 1.8 %) slower than the fastest of the five, at worst 20 % (256 x 4224 x 7552: 35.5 in 128 x 64, 29.6 in 64 x 64),
+// and never slower than 256 x 256. 64 x 128 (15 % faster at 300 x 5120 x 17408, 10 % slower elsewhere) and 128 x 256 (7 %
+// faster at 777 x 5120 x 6144, 9 % slower at 256 x 17408 x 5120) were not worth their kernels.
 enum PrefillTile { kT256x256, kT64x64, kT128x64, kT128x128, kT128x128x2 };  // x2: two stages, two tiles per CU
 PrefillTile choose_tile(const PrefillArgs& a, long long cus) {
   constexpr double kLaunch = 4., kSplit = 10., kPart = 0.07, kBig = 1.72;
@@ -666,6 +673,24 @@ PrefillTile choose_tile(const PrefillArgs& a, long long cus) {
   return tile;
 }
 
+// The 256 x 256 tiles of a product: when they leave the last round of one-tile-per-CU workgroups at most a third full, the
+// tiles of that round are each split along K into S parts (S <= #CUs / rem, each part >= 8 K blocks, S <= 4).
+// Measured on config 4: down (64 of 256 CUs busy in the last round, S = 4) gains 8%; a half-full last round
+// (gate|up, S would be 2) loses 4% to the partial traffic, as the clock rises when CUs idle.
+void split_last_round(PrefillArgs& a, long long cus) {
+  a.KB = a.K / 128;
+  a.tiles_m = cdiv(a.M, kBM);
+  a.tiles_n = cdiv(a.N, kBN);
+  const long long tiles = static_cast<long long>(a.tiles_m) * a.tiles_n;
+  a.rem = static_cast<int>(tiles % cus);
+  a.S = a.rem ? static_cast<int>(std::min<long long>({cus / a.rem, a.KB / 8, kMaxSplit})) : 1;
+  if (a.S < 3) {
+    a.S = 1;
+    a.rem = 0;
+  }
+  a.full = static_cast<int>(tiles - a.rem);
+}
+
 template <bool BLOCK, int OUT>
 int prefill_launch(PrefillArgs a, const char* name, hipStream_t s) {
   const std::string nm(name);
@@ -679,24 +704,10 @@ int prefill_launch(PrefillArgs a, const char* name, hipStream_t s) {
   if (!a.xq || !a.w || !a.y || (BLOCK && (!a.xs || !a.ws))) return fail(LQ_ERR_ARG, nm + ": null pointer");
   if (reinterpret_cast<uintptr_t>(a.y) % (OUT == kOutBf16 ? 8 : 16) != 0)
     return fail(LQ_ERR_ARG, nm + ": y must be 8-byte (BF16) or 16-byte (FP32) aligned");
-  a.KB = a.K / 128;
-  a.tiles_m = cdiv(a.M, kBM);
-  a.tiles_n = cdiv(a.N, kBN);
-  const long long tiles = static_cast<long long>(a.tiles_m) * a.tiles_n;
-  // Tail split: when the tiles leave the last round of one-tile-per-CU workgroups at most a third full, the
-  // tiles of that round are each split along K into S parts (S <= #CUs / rem, each part >= 8 K blocks, S <= 4).
-  // Measured on config 4: down (64 of 256 CUs busy in the last round, S = 4) gains 8%; a half-full last round
-  // (gate|up, S would be 2) loses 4% to the partial traffic, as the clock rises when CUs idle.
   int dev = 0;
   (void)hipGetDevice(&dev);
   const long long P = device_cus(dev);
-  a.rem = static_cast<int>(tiles % P);
-  a.S = a.rem ? static_cast<int>(std::min<long long>({P / a.rem, a.KB / 8, kMaxSplit})) : 1;
-  if (a.S < 3) {
-    a.S = 1;
-    a.rem = 0;
-  }
-  a.full = static_cast<int>(tiles - a.rem);
+  split_last_round(a, P);
   switch (choose_tile(a, P)) {
     case kT64x64: return tile_launch<BLOCK, OUT, 2, 2, 2, 2, 4>(a, name, s);
     case kT128x64: return tile_launch<BLOCK, OUT, 4, 2, 2, 2, 3>(a, name, s);
@@ -738,6 +749,18 @@ int reserve_prefill_scratch(Workspace* ws) {
 using namespace lq;
 
 extern "C" {
+
+// Test hook (not part of the interface): the tile of a product on `cus` CUs, 8 * PrefillTile + the parts along K of a tile
+// of the last round (1: not split).
+int lq_debug_prefill_fp8_tile(int M, int N, int K, int cus) {
+  PrefillArgs a{};
+  a.M = M;
+  a.N = N;
+  a.K = K;
+  split_last_round(a, cus);
+  const PrefillTile tile = choose_tile(a, cus);
+  return 8 * tile + (tile == kT256x256 ? a.S : 1);
+}
 
 int lq_quant_act_fp8_g128(const uint16_t* x, int M, int K, uint8_t* q, float* scale, void* stream) {
   if (M < 1 || K <= 0 || K % 128 != 0) return fail(LQ_ERR_SHAPE, "quant_act_fp8_g128: M >= 1 and K % 128 == 0");

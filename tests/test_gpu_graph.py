@@ -4,6 +4,8 @@ the skinny GEMMs (gate|up + SiLU*mul, down + residual, NVFP4 with BF16 activatio
 several times with new inputs written eagerly between replays; every replay must equal, bit for bit, eager
 launches on the same inputs (split-K counters and partial buffers reset themselves inside the kernels, so no
 replay depends on memory a previous one left)."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -76,8 +78,18 @@ def test_verify_step_and_nvfp4_under_graph_replay(L):
             assert torch.equal(a, b.view(torch.int16)), f"replay {rep}: {name}"
 
 
-def test_block_prefill_under_graph_replay(L):
-    M, N, K = 300, 256, 4096  # a tail-split shape (its partials and arrival counters are in the capture)
+def prefill_parts(L, M, N, K):
+    """The parts along K of a tile of the last round (0: not in 256 x 256 tiles, which alone are split)."""
+    fn = L.lib.lq_debug_prefill_fp8_tile
+    fn.argtypes, fn.restype = [ctypes.c_int] * 4, ctypes.c_int
+    tile, parts = divmod(fn(M, N, K, torch.cuda.get_device_properties(0).multi_processor_count), 8)
+    return 0 if tile else parts
+
+
+# in 64 x 64 tiles, and a tail-split shape (its partials and arrival counters are in the capture)
+@pytest.mark.parametrize("M,N,K,parts", [(300, 256, 4096, 0), (718, 5504, 6144, 3)])
+def test_block_prefill_under_graph_replay(L, M, N, K, parts):
+    assert prefill_parts(L, M, N, K) == parts
     qw, sw = O.quant_fp8_block128(O.normal_f32(111, 0.02, (N, K)))
     tw, ws = L.retile_fp8(to_dev(qw)), to_dev(sw)
     x = torch.empty((M, K), dtype=torch.bfloat16, device=DEV)
@@ -112,7 +124,8 @@ def test_block_prefill_under_graph_replay(L):
 def test_prefill_scratch_is_not_reallocated(L):
     """A graph captured over a tail-split prefill keeps its scratch pointers valid after a larger tail-split shape has
     run eagerly (the library reserves the scratch at its bound once and never reallocates it)."""
-    M, N, K = 300, 256, 4096
+    M, N, K = 977, 2176, 12288
+    assert prefill_parts(L, M, N, K) == 4  # 36 tiles: 144 partials
     qw, sw = O.quant_fp8_block128(O.normal_f32(131, 0.02, (N, K)))
     tw, ws = L.retile_fp8(to_dev(qw)), to_dev(sw)
     x = bf16(132, (M, K))
@@ -134,9 +147,10 @@ def test_prefill_scratch_is_not_reallocated(L):
     ref = torch.empty_like(y)
     run(ref)
     # a larger tail split: more rows and weight rows, so more split tiles than the captured shape
-    N2, M2 = 1024, 700
-    qw2, sw2 = O.quant_fp8_block128(O.normal_f32(133, 0.02, (N2, K)))
-    xq2, xs2 = L.quant_act_fp8_g128(bf16(134, (M2, K)))
+    M2, N2, K2 = 718, 5504, 6144
+    assert prefill_parts(L, M2, N2, K2) == 3  # 66 tiles: 198 partials
+    qw2, sw2 = O.quant_fp8_block128(O.normal_f32(133, 0.02, (N2, K2)))
+    xq2, xs2 = L.quant_act_fp8_g128(bf16(134, (M2, K2)))
     L.prefill_fp8_block(xq2, xs2, L.retile_fp8(to_dev(qw2)), to_dev(sw2), N2)
     torch.cuda.synchronize()
     for rep in range(3):

@@ -6,6 +6,8 @@ error <= 1e-2 with denominator max(|ref|, rms(row)), mean |err| <= 1e-3), at sma
 config-4 shapes on a row subset; plus size-independent properties (row subsets equal the full launch, zero
 rows stay zero, stray columns past N untouched).
 """
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -21,6 +23,27 @@ def L():
     import ling_gemm
     ling_gemm.init()
     return ling_gemm
+
+
+def tile_of(L, hook, *args):
+    """What the library's rule takes for a shape on this device (lq_debug_prefill_fp8_tile, lq_debug_prefill_nvfp4_tile),
+    so that a test of one kernel notices when its shape no longer gets there."""
+    fn = getattr(L.lib, hook)
+    fn.argtypes, fn.restype = [ctypes.c_int] * (len(args) + 1), ctypes.c_int
+    return fn(*args, torch.cuda.get_device_properties(0).multi_processor_count)
+
+
+T256, T64, T128X64, T128, T128X2 = range(5)  # the FP8 tiles, as the hook numbers them
+
+
+def fp8_tile(L, M, N, K):
+    """(tile, parts along K of a tile of the last round)"""
+    return divmod(tile_of(L, "lq_debug_prefill_fp8_tile", M, N, K), 8)
+
+
+def nvfp4_tile(L, swiglu, M, N, K):
+    """(weight tiles of a wave, waves along the tokens)"""
+    return divmod(tile_of(L, "lq_debug_prefill_nvfp4_tile", int(swiglu), M, N, K), 16)
 
 
 def to_dev(a):
@@ -66,7 +89,7 @@ def prefill_case(L, M, N, K, seed):
     return wq, ws, xq, xs, tw
 
 
-# (300, 256, 4096) and (257, 128, 3072): every tile is split along K into 4 / 3 parts (the tail split)
+# (few 256 x 256 tiles: all of these are done in 64 x 64 ones)
 @pytest.mark.parametrize("M,N,K", [(1, 128, 128), (130, 256, 384), (512, 384, 1024), (257, 128, 3072),
                                    (300, 256, 4096)])
 def test_prefill_small_full(L, M, N, K):
@@ -74,16 +97,18 @@ def test_prefill_small_full(L, M, N, K):
     y = L.prefill_fp8_block(to_dev(xq), to_dev(xs), tw, to_dev(ws), N)
     ref = O.prefill_fp8_rows(xq, xs, np.arange(M), wq, ws)
     check(bf16_host(y), ref, f"prefill M={M} N={N} K={K}")
-    # split tiles add their parts in a fixed order: a second launch is bit-identical
+    assert fp8_tile(L, M, N, K) == (T64, 1)
+    # a second launch is bit-identical
     y2 = L.prefill_fp8_block(to_dev(xq), to_dev(xs), tw, to_dev(ws), N)
     assert np.array_equal(bf16_host(y), bf16_host(y2))
 
 
 # one shape for each of the smaller tiles (64 x 64, 128 x 64, 128 x 128 with four and with two stages), with a last
 # token tile of a few rows and fewer, as many and more K blocks than the tile has stages, odd counts among them
-@pytest.mark.parametrize("M,N", [(81, 384), (257, 4224), (513, 4224), (1026, 4224)])
+@pytest.mark.parametrize("M,N,tile", [(81, 384, T64), (257, 4224, T128X64), (513, 4224, T128), (1026, 4224, T128X2)])
 @pytest.mark.parametrize("K", [128, 384, 640])
-def test_prefill_small_tiles(L, M, N, K):
+def test_prefill_small_tiles(L, M, N, tile, K):
+    assert fp8_tile(L, M, N, K) == (tile, 1)
     wq, ws, xq, xs, tw = prefill_case(L, M, N, K, 60 + M)
     y = L.prefill_fp8_block(to_dev(xq), to_dev(xs), tw, to_dev(ws), N)
     rows = np.unique(np.r_[0, 15, 16, 63, 64, M // 2, M - 2, M - 1])
@@ -93,6 +118,46 @@ def test_prefill_small_tiles(L, M, N, K):
     assert np.array_equal(bf16_host(sub), bf16_host(y)[:17])
     yt = L.prefill_gemm_fp8(to_dev(xq), tw, 3.0e-4, N)
     check_f32(yt.cpu().numpy()[rows].astype(np.float64), pt_ref(xq, wq, 3.0e-4, rows), f"per-tensor M={M} N={N} K={K}")
+
+
+# the 256 x 256 tile, its last row of tiles ragged in M and half empty in N: not split (one K block, and several), and the
+# tiles of the last round in three and in four parts along K
+@pytest.mark.parametrize("M,N,K,parts", [(1303, 6016, 128, 1), (783, 10112, 384, 1), (718, 5504, 6144, 3),
+                                         (977, 2176, 12288, 4)])
+def test_prefill_256_tiles(L, M, N, K, parts):
+    assert fp8_tile(L, M, N, K) == (T256, parts)
+    wq, xq, tw = pt_case(L, M, N, K, 160 + parts)
+    rng = np.random.default_rng(161)
+    xs = (rng.random((M, K // 128), dtype=np.float32) + 0.5).astype(np.float32)
+    ws = (rng.random((N // 128, K // 128), dtype=np.float32) + 0.5).astype(np.float32)
+    rows = np.unique(np.r_[0, 15, 16, 63, 64, 255, 256, M // 2, M - 2, M - 1])
+    xd = to_dev(xq)
+    raw = pt_ref(xq, wq, 1.0, rows)
+    unit = float(1.0 / np.sqrt(np.mean(raw[0] * raw[0])))  # outputs of unit size, as the BF16 bounds assume
+    xs *= np.float32(unit)
+    ldy = N + 64
+
+    def canvas(dtype, value):
+        return torch.full((M, ldy), value, dtype=dtype, device=DEV)
+
+    def written(y, value):
+        assert torch.all(y[:, N:] == value)  # nothing past N
+        return y[:, :N].contiguous()
+
+    # block-scaled
+    y = written(L.prefill_fp8_block(xd, to_dev(xs), tw, to_dev(ws), N, y=canvas(torch.bfloat16, 7.0), ldy=ldy), 7.0)
+    check(bf16_host(y)[rows], O.prefill_fp8_rows(xq, xs, rows, wq, ws), f"block M={M} N={N} K={K}")
+    # (split tiles add their parts in a fixed order: a second launch is bit-identical)
+    y2 = L.prefill_fp8_block(xd, to_dev(xs), tw, to_dev(ws), N)
+    assert torch.equal(y.view(torch.int16), y2.view(torch.int16))
+    # per tensor: FP32, added to what is there, BF16
+    ref = (raw[0] * unit, raw[1] * unit)
+    yt = written(L.prefill_gemm_fp8(xd, tw, unit, N, y=canvas(torch.float32, 0.5), ldy=ldy), 0.5)
+    check_f32(yt.cpu().numpy()[rows].astype(np.float64), ref, f"per-tensor M={M} N={N} K={K}")
+    ya = written(L.prefill_gemm_fp8(xd, tw, unit, N, y=canvas(torch.float32, 0.5), ldy=ldy, accumulate=True), 0.5)
+    assert torch.equal(ya, yt + 0.5)
+    yb = written(L.prefill_gemm_fp8_bf16out(xd, tw, unit, N, y=canvas(torch.bfloat16, 5.0), ldy=ldy), 5.0)
+    assert torch.equal(yb.view(torch.int16), yt.to(torch.bfloat16).view(torch.int16))
 
 
 def test_prefill_stray_columns_and_rows(L):
@@ -378,21 +443,51 @@ def test_prefill_nvfp4(L, M, N, K):
     check_f32_tight(b[:, :N].astype(np.float64), ref + 0.5, "nvfp4 prefill accumulate")
 
 
-# one shape for each tile (64 x 64, then 128 x 64, 128 x 128 and 128 x 256), last tiles of a few rows; fewer, as many and more chunks than
-# a K group has waves, with remainders
-@pytest.mark.parametrize("M,N", [(65, 128), (70, 8320), (260, 8320), (1030, 6528)])
-@pytest.mark.parametrize("K", [128, 896, 1152])
-def test_prefill_nvfp4_tiles(L, M, N, K):
-    wv, ws, xq, xs = _nvfp4_operands(L, M, N, K, 140 + M)
-    raw = L.retile_nvfp4(to_dev(wv), to_dev(ws))
-    y = L.prefill_gemm_nvfp4(to_dev(xq), to_dev(xs), raw, 0.37, N).cpu().numpy()
+def _random_nvfp4(rng, rows, K):
+    """Any codes, 40 scales over a range of 2^5 (few enough for the coded blob)."""
+    return (rng.integers(0, 256, (rows, K // 2), dtype=np.uint8), rng.integers(0x28, 0x50, (rows, K // 16), dtype=np.uint8))
+
+
+# one shape for each tile of the plain form (half and whole wave tiles with eight waves along K, then four), last tiles of a
+# few rows; of K's chunks one, fewer than the waves that share them, as many, and more with a remainder. SwiGLU takes four
+# waves at the third matrix and at K below 896.
+@pytest.mark.parametrize("M,N,tile", [(65, 128, (4, 1)), (1700, 640, (8, 1)), (70, 6528, (8, 2))])
+@pytest.mark.parametrize("K", [128, 384, 512, 896, 1024, 1152])
+def test_prefill_nvfp4_tiles(L, M, N, tile, K):
+    assert nvfp4_tile(L, False, M, N, K) == tile
+    assert nvfp4_tile(L, True, M, N, K) == ((8, 2) if N == 6528 or K < 896 else (8, 1))
+    rng = np.random.default_rng(M + K)
+    (gv, gs), (uv, us), (xq, xs) = (_random_nvfp4(rng, n, K) for n in (N, N, M))
+    gate, up = L.retile_nvfp4(to_dev(gv), to_dev(gs)), L.retile_nvfp4(to_dev(uv), to_dev(us))
+    xqd, xsd = to_dev(xq), to_dev(xs)
     rows = np.unique(np.r_[0, 15, 16, 63, 64, M // 2, M - 2, M - 1])
-    check_f32_tight(y[rows].astype(np.float64), O.prefill_nvfp4_rows(xq, xs, rows, wv, ws, 0.37), f"M={M} N={N} K={K}")
-    # gate = up = the same matrix: the FFN entry against this call's outputs and the quantizer
-    q, sf = L.prefill_swiglu_nvfp4(to_dev(xq), to_dev(xs), raw, 0.37, raw, 0.37, N, 0.05)
-    rq, rsf = L.silu_mul_quant_nvfp4(to_dev(y), to_dev(y), 0.05)
+    raw = O.prefill_nvfp4_rows(xq, xs, rows, gv, gs, 1.0)
+    ag = float(1.0 / np.sqrt(np.mean(raw * raw)))
+    au = 1.7 * ag
+
+    def coded(v, sc):
+        ok, _, code_of = O.scale_code_table(sc)
+        assert ok
+        return L.retile_nvfp4_coded(to_dev(v), to_dev(sc), to_dev(code_of))
+
+    (gc, gr), (uc, ur) = coded(gv, gs), coded(uv, us)
+    g = L.prefill_gemm_nvfp4(xqd, xsd, gate, ag, N)
+    check_f32_tight(g.cpu().numpy()[rows].astype(np.float64), ag * raw, f"M={M} N={N} K={K}")
+    # the coded blob with its raw scales: the same bits
+    assert torch.equal(L.prefill_gemm_nvfp4(xqd, xsd, gc, ag, N, wsf=gr), g)
+    # added to rows ldy apart
+    ldy = N + 32
+    base = torch.full((M, ldy), 0.5, dtype=torch.float32, device=DEV)
+    L.prefill_gemm_nvfp4(xqd, xsd, gate, ag, N, y=base, ldy=ldy, accumulate=True)
+    assert torch.all(base[:, N:] == 0.5) and torch.equal(base[:, :N], g + 0.5)
+    # the FFN entry of two different matrices against their products and the quantizer
+    u = L.prefill_gemm_nvfp4(xqd, xsd, up, au, N)
+    q, sf = L.prefill_swiglu_nvfp4(xqd, xsd, gate, ag, up, au, N, 0.05)
+    rq, rsf = L.silu_mul_quant_nvfp4(g, u, 0.05)
     # (the same sums in another K split can move a value across a rounding boundary)
     assert (q != rq).float().mean().item() <= 3e-3 and (sf != rsf).float().mean().item() <= 1e-3
+    q2, sf2 = L.prefill_swiglu_nvfp4(xqd, xsd, gc, ag, uc, au, N, 0.05, gate_sf=gr, up_sf=ur)
+    assert torch.equal(q2, q) and torch.equal(sf2, sf)
 
 
 # matrices with eight waves along K (SwiGLU; plain, in both weight tiles) and with four
