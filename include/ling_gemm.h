@@ -182,13 +182,14 @@ int lq_stream_nvfp4_bf16(const uint16_t* x, int M, const uint8_t* w, const uint8
 /* ---------------- prefill, NVFP4 (reference src/core/kernels.cuh:207-221) ---------------- */
 /* y[M][0..N) (rows ldy apart, FP32) = alpha * xq . W^T, or += with accumulate; xq NVFP4 activations [M][K/2] with E4M3
  * block scales xs [M][K/16]; W the tiled NVFP4 blob (raw; or coded with wsf = its raw scales, 128 B per block).
- * Both operands are dequantized exactly (E2M1 x E4M3) and multiplied in FP32. N % 128 == 0, K % 128 == 0; M < 1
- * does nothing. kernels.cuh:210-211 prefill_gemm_nvfp4. */
+ * Both operands are dequantized exactly (E2M1 x E4M3) and multiplied in FP32. A row's result has the same bits at any
+ * M. N % 128 == 0, K % 128 == 0; M < 1 does nothing. kernels.cuh:210-211 prefill_gemm_nvfp4. */
 int lq_prefill_gemm_nvfp4(const uint8_t* xq, const uint8_t* xs, int M, const uint8_t* w, float alpha, float* y, int ldy,
                           int N, int K, int accumulate, void* stream, const uint8_t* wsf);
 /* The FFN's gate and up projections into the down projection's input: NVFP4 of BF16(silu(alpha_gate * xq . G^T) *
  * (alpha_up * xq . U^T)) with global scale 1 / out_input_scale, q_out [M][N/2], sf_out [M][N/16]; gate_sf / up_sf:
- * raw scales of coded blobs (both or neither). N % 128 == 0, K % 128 == 0. kernels.cuh:217-221 prefill_swiglu_nvfp4. */
+ * raw scales of coded blobs (both or neither). A row's result has the same bits at any M. N % 128 == 0, K % 128 == 0.
+ * kernels.cuh:217-221 prefill_swiglu_nvfp4. */
 int lq_prefill_swiglu_nvfp4(const uint8_t* xq, const uint8_t* xs, int M, const uint8_t* gate, float alpha_gate,
                             const uint8_t* up, float alpha_up, int N, int K, float out_input_scale, uint8_t* q_out,
                             uint8_t* sf_out, void* stream, const uint8_t* gate_sf, const uint8_t* up_sf);
@@ -220,7 +221,8 @@ int lq_rmsnorm_quant_bf16(const float* x, const uint16_t* w, uint16_t* out, int 
 int lq_quant_act_fp8_g128(const uint16_t* x, int M, int K, uint8_t* q, float* scale, void* stream);
 /* y[M][0..N) (rows ldy apart, BF16) = bf16(sum over 128-value K blocks kb of (xq . W^T over kb) * xs[m][kb] *
  * ws[n/128][kb]); xq FP8 [M][K], xs FP32 [M][K/128], W tiled FP8 (the stream GEMMs' blob), ws FP32 [N/128][K/128].
- * N % 128 == 0, K % 128 == 0; M < 1 does nothing. The block-scaled, BF16-out form of prefill_gemm_fp8
+ * N % 128 == 0, K % 128 == 0; M < 1 does nothing. Deterministic; a row's last bits can differ between calls of different
+ * M, which decides where FP8 prefill calls split K (per tensor too). The block-scaled, BF16-out form of prefill_gemm_fp8
  * (kernels.cuh:213-214) and prefill_gemm_fp8_bf16out (kernels.cuh:239-240). */
 int lq_prefill_fp8_block(const uint8_t* xq, const float* xs, int M, const uint8_t* w, const float* ws, uint16_t* y,
                          int ldy, int N, int K, void* stream);
