@@ -31,11 +31,10 @@ LQ_HOST_DEVICE inline unsigned activation_unit_offset(int m, int u, int K) {
 LQ_HOST_DEVICE inline unsigned block_offset(int kb, int KB, int step) {
   return static_cast<unsigned>(kb < KB ? kb : KB - 1) * static_cast<unsigned>(step);
 }
-// Scalar offset, without its K block, of load i of a wave whose rows lie `step` bytes (64 rows) apart from load to load, the
-// first of load 0 being `row`: load 0's rows again where an operand of `rows` has none of load i's, since an offset past its
-// end must not be (what such rows give is never stored).
-LQ_HOST_DEVICE inline unsigned load_offset(int row, int i, int rows, unsigned step) {
-  return row + 64 * i < rows ? static_cast<unsigned>(i) * step : 0u;
-}
+// The 256 x 256 tile issues its loads for all its rows, there or not: load i (0 .. 3) of a wave is 64 i rows on, by the scalar
+// offset. For loads 0 to 2 that is within an operand of kWholeRows rows; load 3 of fewer than 193, which has no rows then,
+// repeats load 0's (what such rows give is never stored). Weights have 256 rows or more.
+constexpr int kWholeRows = 129;
+LQ_HOST_DEVICE inline unsigned last_load_offset(int rows, unsigned step) { return rows > 192 ? 3u * step : 0u; }
 
 }  // namespace lq

@@ -31,6 +31,7 @@
 #include "lq_workspace.hpp"
 
 #include <algorithm>
+#include <limits>
 #include <string>
 #include <type_traits>
 
@@ -168,15 +169,12 @@ __global__ void __launch_bounds__(kThreads) prefill_fp8_kernel(const PrefillArgs
   // Load-to-LDS plan: load i (0..3) of wave w writes LDS bytes [((i * 8 + w) * 64 + lane) * 16, +16) of an
   // operand tile: row = (i * 8 + w) * 8 + lane / 8, swizzled unit lane % 8, i.e. source unit u = lane % 8 ^ swz(row)
   // (the same for every i, as i moves the row by 64, a multiple of 16). The per-i and per-block steps go in the scalar
-  // offset.
+  // offset, which stays within the operands (lq_prefill_offsets.hpp; choose_tile gives ones of fewer than kWholeRows rows to
+  // the other tiles).
   const int row0 = wave * 8 + (lane >> 3), u0 = (lane & 7) ^ swz(row0);
   const unsigned wsrc = weight_unit_offset(n0 + row0, u0, a.KB), xsrc = activation_unit_offset(m0 + row0, u0, a.K);
-  unsigned wload[4], xload[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    wload[i] = load_offset(n0 + wave * 8, i, a.N, 64u * static_cast<unsigned>(a.K));
-    xload[i] = load_offset(m0 + wave * 8, i, a.M, 64u * static_cast<unsigned>(a.K));
-  }
+  const unsigned step = 64u * static_cast<unsigned>(a.K);  // 64 rows, of either operand
+  const unsigned xlast = last_load_offset(a.M, step);
   // activation scales: waves 0-3 load one token's scale per lane
   const int srow = wave * 64 + lane;
   const int ssrc = (wave < 4 && m0 + srow < a.M) ? (m0 + srow) * a.KB * 4 : static_cast<int>(0x80000000u);
@@ -188,11 +186,11 @@ __global__ void __launch_bounds__(kThreads) prefill_fp8_kernel(const PrefillArgs
     if (part < 2) {
 #pragma unroll
       for (int i = 2 * part; i < 2 * part + 2; ++i)
-        dma16(wr, base + (i * 8 + wave) * 1024, wsrc, kb * kTileBytesFp8 + wload[i]);
+        dma16(wr, base + (i * 8 + wave) * 1024, wsrc, kb * kTileBytesFp8 + i * step);
     } else if (part < 4) {
 #pragma unroll
       for (int i = 2 * (part - 2); i < 2 * (part - 2) + 2; ++i)
-        dma16(xr, base + kOpBytes + (i * 8 + wave) * 1024, xsrc, kb * kRowBytes + xload[i]);
+        dma16(xr, base + kOpBytes + (i * 8 + wave) * 1024, xsrc, kb * kRowBytes + (i < 3 ? i * step : xlast));
     } else if (BLOCK && wave < 4) {
       dma4(sr, base + 2 * kOpBytes + wave * 256, ssrc, kb * 4);
     }
@@ -639,7 +637,8 @@ int tile_launch(PrefillArgs a, const char* name, hipStream_t s) {
 // (microseconds, weights from memory), `pair` what one of two resident tiles' costs together; the larger the tile, the
 // less each output costs, but tiles come in whole numbers per CU, so a product with few of them is done sooner in
 // smaller ones. A launch costs 4 us; a split last round of 256 x 256 tiles 10 us more and 0.07 us per part, for the
-// exchange. The smallest sum wins, the 256 x 256 tile unless another is 5 % better. Measured, block-scaled (M x N x K,
+// exchange. The smallest sum wins, the 256 x 256 tile unless another is 5 % better or an operand has too few rows for its
+// loads' offsets (kWholeRows). Measured, block-scaled (M x N x K,
 // us, rotating over 500 MB of weights): 200 x 2048 x 4096 32 -> 12 (64 x 64), 200 x 7168 x 5120 42 -> 22 (128 x 64),
 // 300 x 5120 x 17408 83 -> 72 (128 x 64), 512 x 5120 x 5120 45 -> 34 (128 x 128), 1500 x 5120 x 17408 238 -> 153 (128 x 128
 // x2); 1000 x 5120 x 17408 stays at 114 (133 in 128 x 128 x2) and 500 x 17408 x 5120 at 83 (80 in 128 x 128 x2).
@@ -655,6 +654,7 @@ PrefillTile choose_tile(const PrefillArgs& a, long long cus) {
   double best = kLaunch + a.KB * kBig * static_cast<double>((a.full + cus - 1) / cus);
   if (a.rem) best += kBig * a.KB / a.S + kSplit + kPart * a.rem * a.S;
   best *= 0.95;
+  if (a.M < kWholeRows || a.N < 256) best = std::numeric_limits<double>::infinity();
   PrefillTile tile = kT256x256;
   struct Kind {
     PrefillTile tile;

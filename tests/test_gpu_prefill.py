@@ -120,10 +120,10 @@ def test_prefill_small_tiles(L, M, N, tile, K):
     check_f32(yt.cpu().numpy()[rows].astype(np.float64), pt_ref(xq, wq, 3.0e-4, rows), f"per-tensor M={M} N={N} K={K}")
 
 
-# the 256 x 256 tile, its last row of tiles ragged in M and half empty in N: not split (one K block, and several), and the
-# tiles of the last round in three and in four parts along K
-@pytest.mark.parametrize("M,N,K,parts", [(1303, 6016, 128, 1), (783, 10112, 384, 1), (718, 5504, 6144, 3),
-                                         (977, 2176, 12288, 4)])
+# the 256 x 256 tile, its last row of tiles ragged in M and half empty in N: not split (one K block, and several; with fewer
+# tokens than its last load's first row), and the tiles of the last round in three and in four parts along K
+@pytest.mark.parametrize("M,N,K,parts", [(160, 48768, 384, 1), (1303, 6016, 128, 1), (783, 10112, 384, 1),
+                                         (718, 5504, 6144, 3), (977, 2176, 12288, 4)])
 def test_prefill_256_tiles(L, M, N, K, parts):
     assert fp8_tile(L, M, N, K) == (T256, parts)
     wq, xq, tw = pt_case(L, M, N, K, 160 + parts)

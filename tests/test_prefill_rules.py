@@ -42,3 +42,16 @@ def test_nvfp4_choices_as_measured(L, swiglu, M, N, K, tile):
     (4096, 5120, 17408, 0, 4)])
 def test_fp8_choices_as_measured(L, M, N, K, tile, parts):
     assert divmod(L.lq_debug_prefill_fp8_tile(M, N, K, 256), 8) == (tile, parts)
+
+
+@pytest.mark.parametrize("cus", [256, 64, 8])
+def test_256_tiles_only_where_their_offsets_stay_within_the_operands(L, cus):
+    """The 256 x 256 tile's scalar offsets need 129 tokens and 256 weight rows."""
+    taken = 0
+    for M in (1, 17, 64, 81, 128, 129, 192, 256, 1000, 100000):
+        for N in (128, 256, 384, 5120, 34816, 151936):
+            for K in (128, 1024, 5120, 17408):
+                whole = L.lq_debug_prefill_fp8_tile(M, N, K, cus) // 8 == 0
+                assert not whole or (M >= 129 and N >= 256), f"{M} x {N} x {K}"
+                taken += whole
+    assert taken
