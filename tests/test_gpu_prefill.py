@@ -130,7 +130,7 @@ def test_prefill_256_tiles(L, M, N, K, parts):
     rng = np.random.default_rng(161)
     xs = (rng.random((M, K // 128), dtype=np.float32) + 0.5).astype(np.float32)
     ws = (rng.random((N // 128, K // 128), dtype=np.float32) + 0.5).astype(np.float32)
-    rows = np.unique(np.r_[0, 15, 16, 63, 64, 255, 256, M // 2, M - 2, M - 1])
+    rows = np.unique(np.r_[0, 15, 16, 63, 64, 127, 128, min(255, M - 3), min(256, M - 3), M // 2, M - 2, M - 1])
     xd = to_dev(xq)
     raw = pt_ref(xq, wq, 1.0, rows)
     unit = float(1.0 / np.sqrt(np.mean(raw[0] * raw[0])))  # outputs of unit size, as the BF16 bounds assume
