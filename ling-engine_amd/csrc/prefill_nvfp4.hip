@@ -25,8 +25,7 @@
 //    13.5 KB of LDS by direct loads, takes a landed chunk into registers (60 of them) and at once has the next one loaded
 //    over it, which then has the whole chunk's 128 MFMAs to arrive.
 //  * LDS of a wave (NI = 8): [weight values 128 x 64 B][weight scales 128 x 8][token values 64 x 64][token scales 64 x 8]. The
-//    16-byte units of a 64-byte row are XOR-swizzled by swz4(row) so the 16-byte fragment reads are conflict free whether
-//    the LDS serves 8 or 16 lanes of them per cycle; four lanes of a load read one run of 64 bytes.
+//    16-byte units of a 64-byte row are XOR-swizzled by swz4(row); four lanes of a load read one run of 64 bytes.
 //
 // What bounds it: the dequantization and the MFMAs share the SIMD's issue (3 VALU instructions per MFMA). Tiles of 256 x
 // 256 over 8 waves, which read a step's word from LDS just ahead of its use, took 430 us at 300 x 5120 x 17408 (40 tiles
@@ -43,8 +42,10 @@ constexpr int wave_off_x(int ni) { return ni * 16 * 72; }  // a wave's LDS: 16 n
 constexpr int kRedWave = 16 * 1024;  // a wave's sums of four weight tiles x four token tiles
 static_assert(kRedWave >= wave_off_x(8) + 64 * 72, "the reduction takes the larger part of LDS");
 
-// 16 lanes read one 16-byte unit each of rows r .. r + 15 (r % 16 == 0): banks (row % 4, unit) must be distinct
-// over the 16 rows, and (row % 2, unit) over each aligned 8.
+// Lane (r, t) reads unit t of row r, 16 bytes. 16 lanes of one t have no bank conflict, but the LDS serves rows 0-3 and 12-15 of
+// one t with rows 4-11 of the next, where every read is a two-way one (3-5 % of the CUs' cycles). They are hidden: a swizzle
+// without any (units of rows 0-3, 4-7, 8-11, 12-15 by 0, 2, 3, 1; counted 0) took 63.9 us at 300 x 5120 x 17408, this one 63.6,
+// and the same at 2048 x 17408 x 5120 SwiGLU.
 __device__ __forceinline__ int swz4(int row) { return ((row >> 1) & 3) ^ ((row >> 3) & 1); }
 __device__ __forceinline__ int val_off(int row, int u) { return row * 64 + ((u ^ swz4(row)) << 4); }
 
