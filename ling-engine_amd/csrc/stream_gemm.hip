@@ -17,8 +17,8 @@
 //    is applied in FP32 in the epilogue.
 //  * A workgroup is 4 waves over a tile group of 16 tiles (256 weight rows); wave w owns tiles
 //    4w .. 4w + 3 and all waves walk the same K chunks in lock step. Each chunk's activations are staged
-//    once per workgroup in LDS (each wave loads a quarter; 16-byte units XOR-swizzled by row so the
-//    MFMA operand reads are conflict free), while each wave streams its own weights through a ring of PF
+//    once per workgroup in LDS (each wave loads a quarter; 16-byte units XOR-swizzled by row,
+//    xs_off), while each wave streams its own weights through a ring of PF
 //    chunks in registers. Loads retire in issue order, so a chunk's activation share is issued before its
 //    weights and the stages are consumed oldest first: every wait leaves the newer stages in flight.
 //  * Work split: units = (tile group, K chunk); P workgroups each take a contiguous, equal range of
