@@ -52,7 +52,10 @@ constexpr int kStage = 2 * kOpBytes + kBM * 4;   // weights, activations, activa
 // swizzles agree on is that the LDS serves such a read 16 lanes at a time, lanes 0-3, 12-15, 20-23 and 24-27 of each 32 and
 // then the others: rows 0-3 and 12-15 of one t with rows 4-11 of the next. So swz serves reads of unit 2t or 2t + 1, swz_w those of
 // unit t or 4 + t, each with no conflict, and also if 8 or 16 lanes in a row were served together; reads of unit t under
-// swz are two-way conflicts, as those of unit 2t under a swizzle by row / 2 are (half of all LDS cycles).
+// swz are two-way conflicts, as those of unit 2t under a swizzle by row / 2 are (half of all LDS cycles). Weights under
+// swz_w are faster in the 256 x 256 tile (1000 x 5120 x 17408 110.2 -> 108.1 us, 2048 x 7168 x 5120 82.7 -> 81.8), under swz in the
+// smaller ones, where the conflicts are hidden and swz_w costs more than it saves, in its loads (428 x 7168 x 5120 28.7, 29.2
+// us, 1500 x 2048 x 4096 22.0, 23.2; three more swizzles without conflicts likewise).
 __device__ __forceinline__ int swz(int row) { return (row & 7) ^ ((row >> 3) & 1); }
 __device__ __forceinline__ int swz_w(int row) {
   return ((((row >> 2) ^ (row >> 3)) & 1) << 2) | (((row >> 3) & 1) << 1) | ((row >> 1) & 1);
@@ -68,8 +71,9 @@ __device__ __forceinline__ i32x8 fragment(const uint8_t* op, int row, int u0, in
   const u32x4 hi = *reinterpret_cast<const u32x4*>(op + lds_off(row, u1));
   return i32x8{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
 }
-__device__ __forceinline__ i32x8 fragment_w(const uint8_t* op, int row, int t) {
-  return fragment(op, row, t ^ swz_w(row), (4 + t) ^ swz_w(row));
+// sw: the weights' swizzle of the row, swz_w (256 x 256 tile) or swz.
+__device__ __forceinline__ i32x8 fragment_w(const uint8_t* op, int row, int t, int sw) {
+  return fragment(op, row, t ^ sw, (4 + t) ^ sw);
 }
 __device__ __forceinline__ i32x8 fragment_x(const uint8_t* op, int row, int t) {
   return fragment(op, row, (2 * t) ^ swz(row), (2 * t + 1) ^ swz(row));
@@ -226,7 +230,7 @@ __global__ void __launch_bounds__(kThreads) prefill_fp8_kernel(const PrefillArgs
   auto block_start = [&](int st) {
     const uint8_t* sa = smem + st * kStage;
     const float* sxs = reinterpret_cast<const float*>(sa + 2 * kOpBytes);
-    af = fragment_w(sa, wn * 128 + r, t);
+    af = fragment_w(sa, wn * 128 + r, t, swz_w(r));
 #pragma unroll
     for (int j = 0; j < 4; ++j) bf[j] = fragment_x(sa + kOpBytes, wm * 64 + 16 * j + r, t);
     if constexpr (BLOCK) {
@@ -276,7 +280,7 @@ __global__ void __launch_bounds__(kThreads) prefill_fp8_kernel(const PrefillArgs
         asm volatile("" ::"v"(acc[i][0]), "v"(acc[i][1]), "v"(acc[i][2]), "v"(acc[i][3]) : "memory");
       __builtin_amdgcn_s_setprio(0);
       if (i < 7) {
-        af = fragment_w(sa, wn * 128 + 16 * (i + 1) + r, t);
+        af = fragment_w(sa, wn * 128 + 16 * (i + 1) + r, t, swz_w(r));
       } else {
         // every wave's reads of this stage have returned and its loads of the next block have landed
         LQ_WAIT_LGKM0();
@@ -410,7 +414,7 @@ __global__ void __launch_bounds__(64 * WN * WM) prefill_tile_kernel(const Prefil
   unsigned wsrc[LW], xsrc[LX], ssrc = kLoadNothing;
 #pragma unroll
   for (int i = 0; i < LW; ++i) {
-    const int row = (i * NW + wave) * 8 + (lane >> 3), u = (lane & 7) ^ swz_w(row), n = n0 + row;
+    const int row = (i * NW + wave) * 8 + (lane >> 3), u = (lane & 7) ^ swz(row), n = n0 + row;
     wsrc[i] = n < a.N ? weight_unit_offset(n, u, a.KB) : kLoadNothing;
   }
 #pragma unroll
@@ -464,7 +468,7 @@ __global__ void __launch_bounds__(64 * WN * WM) prefill_tile_kernel(const Prefil
         f.ws = scalar_load(wsrow + min(kb, a.KB - 1));
       }
     }
-    f.a[i] = fragment_w(sa, wn * NI * 16 + 16 * i + r, t);
+    f.a[i] = fragment_w(sa, wn * NI * 16 + 16 * i + r, t, swz(r));
 #pragma unroll
     for (int j = i * NJ / NI; j < (i + 1) * NJ / NI; ++j) f.b[j] = fragment_x(sa + TN * kRowBytes, wm * NJ * 16 + 16 * j + r, t);
   };
