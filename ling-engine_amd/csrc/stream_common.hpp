@@ -141,8 +141,8 @@ __device__ __forceinline__ void load_w(WRegs<WF, T>& R, const __amdgpu_buffer_rs
 // loaded and stored with the chunk's activations, a chunk ahead of their use. (Loaded by the lanes that use them they were
 // four 2-byte loads per chunk, coded eight of one byte, on the path that the weight stream shares: coded 17408 x 5120 at
 // M = 1 20.4 -> 18.5 us, 5120 x 25600 at M = 16 25.6 -> 22.5; raw 16.8 -> 16.5 and 20.4 -> 20.0 at M = 16. Raw scales
-// beside an FP16 row copy of 17 to 32 rows stay with the lanes:
-// 5120 x 25600 at M = 17, 24, 32 25.5, 25.8, 25.9 us, through LDS 26.3, 26.7, 26.8; 17408 x 5120 22.0, 22.2, 23.2 and 22.4, 22.7, 23.7.)
+// beside an FP16 row copy of 17 to 32 rows stay with the lanes: 5120 x 25600 at M = 17, 24, 32 25.5, 25.8, 25.9 us, through
+// LDS 26.3, 26.7, 26.8; 17408 x 5120 22.0, 22.2, 23.2 and 22.4, 22.7, 23.7.)
 __device__ __forceinline__ u32x2 load_scales(const __amdgpu_buffer_rsrc_t& rs, int soff, int lane_off, unsigned oob) {
   return __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rs, static_cast<int>(lane_off | oob), soff, 0));
 }
